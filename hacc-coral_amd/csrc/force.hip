@@ -59,6 +59,9 @@ struct Item {
   int64_t pbase;    // partial-force offset (-1: write F directly)
 };
 
+// Degree of the fitted grid force's polynomial in r (fit_poly).
+constexpr int FITN = 15;
+
 struct LawArgs {
   float c[7];      // polynomial in s (degree 5 or 6)
   float rcs;       // s cutoff: pairs with s < rcs contribute
@@ -73,26 +76,22 @@ struct LawArgs {
   // ForceLawSR with FGridEvalFit or FGridEvalInterp: f = s^-3/2 - g(r2),
   // pairs with r2 < rc2 contribute
   float rc2;
-  float b, cc, d, e, ff, g, h, l, rmax, f0;  // FGrid constants (ForceLaw.cxx:23-33)
+  float fit[FITN + 1];  // FGrid::fgor as a polynomial in t = fit_a r - 1
+  float fit_a;          // 2 / rmax
   const float4 *bins;                        // {r2[i], f[i], f[i+1] - f[i], 0}
   float t_r2min, t_r2max, t_oodr2;
   int t_last;                                // last bin index (n_interp - 2)
 };
 
-// FGrid::fgor(r), the fitted grid force over r (ForceLaw.cxx:39-51), in
-// float with the device's coshf, tanhf and expf (the reference mixes a few
-// double products in; the difference is a rounding of fgor, far inside the
-// force tolerance).  Entries padded far away keep every term finite.
+// FGrid::fgor(r), the fitted grid force over r (ForceLaw.cxx:39-51), for r in
+// [0, rmax]: the polynomial of fit_poly by Horner's rule.  Beyond rmax it is
+// meaningless (the pair is masked by a select).
 __device__ __forceinline__ float fgor_fit(const LawArgs &L, float r) {
-  const float r2 = r * r, r4 = r2 * r2, r6 = r4 * r2;
-  const float br = L.b * r;
-  const float ch = coshf(br);
-  const float t = tanhf(br) - br / ch / ch +
-                  L.cc * r * r2 * (1.f + L.d * r2) * expf(-L.d * r2) +
-                  L.e * r2 * (L.ff * r2 + L.g * r4 + L.l * r6) * expf(-L.h * r2);
-  const float rdiv = r + (r <= 0.f ? 1.f : 0.f);
-  const float v = t / (rdiv * rdiv * rdiv) + (r <= 0.f ? L.f0 : 0.f);
-  return (r <= L.rmax && r >= 0.f) ? v : 0.f;
+  const float t = fmaf(r, L.fit_a, -1.f);
+  float q = L.fit[FITN];
+#pragma unroll
+  for (int k = FITN - 1; k >= 0; --k) q = fmaf(q, t, L.fit[k]);
+  return q;
 }
 
 // FGridEvalInterp::eval(r2) (ForceLaw.cxx:160-171): linear interpolation in
@@ -194,12 +193,14 @@ __device__ __forceinline__ void pair(const LawArgs &L, float c0, float rcs, cons
     const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
     const float s = r2 + L.eps2;
     const float y = __builtin_amdgcn_rsqf(s);
-    const float gr = LAWK == LAWK_FIT ? fgor_fit(L, __builtin_sqrtf(r2)) : fgor_interp(L, r2);
+    const float gr = LAWK == LAWK_FIT ? fgor_fit(L, __builtin_amdgcn_sqrtf(r2)) : fgor_interp(L, r2);
     f = y * y * y - gr;
     if constexpr (MASKED) {
-      float mm = (r2 < L.rc2) ? p.w : 0.f;
-      if (GUARD) mm = (r2 > 0.f) ? mm : 0.f;
-      f *= mm;
+      // a select, not a product: the fit's polynomial overflows at the padding
+      // entries' distance
+      bool in = r2 < L.rc2;
+      if (GUARD) in = in && r2 > 0.f;
+      f = in ? f * p.w : 0.f;
     }
   }
   ax = fmaf(f, dx, ax);
@@ -530,6 +531,64 @@ hsr_status excl_scan(hsr_ctx *c, const T *in, T *out, int64_t n) {
   return HSR_OK;
 }
 
+// FGrid::fgor(r) = [tanh(br) - br/cosh^2(br) + cc r^3 (1 + d r^2) e^(-d r^2) +
+// e r^2 (ff r^2 + g r^4 + l r^6) e^(-h r^2)] / r^3 on [0, rmax]
+// (ForceLaw.cxx:23-51) as a polynomial of degree FITN in t = 2 r / rmax - 1:
+// its interpolant at the Chebyshev points of the first kind, in double.
+//
+// fgor is analytic in r -- the first term's nearest singularities are the
+// poles of tanh at r = +-i pi / (2 b) -- so the interpolants converge
+// geometrically (about 3.6x per degree); at degree 15 the interpolant is
+// within 2.4e-9 of fgor, below the float rounding of Horner's rule (3.6e-8
+// at most, 7e-9 rms, against 0.26 at r = 0).  The expression itself in float
+// loses up to 7e-5 for r > 0.05 and everything below r = 1e-3, where its
+// first two terms cancel, and costs a coshf, a tanhf, two expf and three
+// divisions per pair.  The pair is bound by VALU issue: 16 FMA and a square
+// root in place of these took the leaf kernel from 6.88 to 1.00 ms on a
+// 60^3 Plummer mix (216k particles, leaves of 128, 3.1e8 pairs).
+void fit_poly(float *out, float *scale) {
+  const double b = 0.72f, cc = 0.01f, d = 0.27f, e = 0.0001f, ff = 360.0f, g = 100.0f, h = 0.67f,
+               l = 17.0f, rmax = 3.116326355f;
+  auto fgor = [&](double r) {
+    const double r2 = r * r, u = b * r, u2 = u * u;
+    // (tanh u - u / cosh^2 u) / u^3: from tanh's series where the terms cancel
+    double th;
+    if (u < 0.1) {
+      th = 2.0 / 3.0 - u2 * (8.0 / 15.0 - u2 * (34.0 / 105.0 - u2 * (496.0 / 2835.0 -
+           u2 * (13820.0 / 155925.0))));
+    } else {
+      const double ch = std::cosh(u);
+      th = (std::tanh(u) - u / (ch * ch)) / (u2 * u);
+    }
+    return b * b * b * th + cc * (1.0 + d * r2) * std::exp(-d * r2) +
+           e * r * (ff + g * r2 + l * r2 * r2) * std::exp(-h * r2);
+  };
+  constexpr int n = FITN + 1;
+  const double pi = std::acos(-1.0);
+  double cheb[n], mono[n] = {}, tp[n] = {}, tc[n] = {}, tn[n];
+  double f[n];
+  for (int i = 0; i < n; ++i) f[i] = fgor(0.5 * rmax * (std::cos(pi * (i + 0.5) / n) + 1.0));
+  for (int k = 0; k < n; ++k) {
+    cheb[k] = 0.0;
+    for (int i = 0; i < n; ++i) cheb[k] += f[i] * std::cos(pi * k * (i + 0.5) / n);
+    cheb[k] *= (k == 0 ? 1.0 : 2.0) / n;
+  }
+  // T_0 = 1, T_1 = t, T_(k+1) = 2 t T_k - T_(k-1), summed into powers of t
+  tp[0] = 1.0;
+  tc[1] = 1.0;
+  for (int i = 0; i < n; ++i) mono[i] = cheb[0] * tp[i] + cheb[1] * tc[i];
+  for (int k = 2; k < n; ++k) {
+    for (int i = 0; i < n; ++i) tn[i] = (i ? 2.0 * tc[i - 1] : 0.0) - tp[i];
+    for (int i = 0; i < n; ++i) {
+      mono[i] += cheb[k] * tn[i];
+      tp[i] = tc[i];
+      tc[i] = tn[i];
+    }
+  }
+  for (int i = 0; i < n; ++i) out[i] = (float)mono[i];
+  *scale = (float)(2.0 / rmax);
+}
+
 // P(r2) = sum a_k r2^k re-expanded in s = r2 + eps2 (host, double).
 LawArgs law_args(const ForceLawDev &D) {
   LawArgs A;
@@ -563,10 +622,7 @@ LawArgs law_args(const ForceLawDev &D) {
   A.in2 = (float)((double)D.rc2 * (1.0 - 1e-4));
   A.unmasked = D.guard ? 0 : 1;
   A.rc2 = D.rc2;
-  // FGrid (ForceLaw.cxx:23-33); f0 = c + 2/3 b^3 as the reference rounds it
-  A.b = 0.72f; A.cc = 0.01f; A.d = 0.27f; A.e = 0.0001f; A.ff = 360.0f; A.g = 100.0f;
-  A.h = 0.67f; A.l = 17.0f; A.rmax = 3.116326355f;
-  A.f0 = (float)(A.cc + 2.0 / 3.0 * A.b * A.b * A.b);
+  fit_poly(A.fit, &A.fit_a);
   A.bins = D.bins;
   A.t_r2min = D.t_r2min;
   A.t_r2max = D.t_r2max;
