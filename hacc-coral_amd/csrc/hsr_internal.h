@@ -140,9 +140,7 @@ struct ListState {
   int64_t plan_stride = 0;    // per-leaf plan arrays' stride (grows only)
   int64_t *multi = nullptr, *counts = nullptr, *leaf_pbase = nullptr;
   int32_t *leaf_nchunk = nullptr;
-  DBuf stack;                 // DFS stacks
-  DBuf walk;                  // per (leaf, sibling walk): counts and offsets
-  DBuf segcache;              // the first segments each walk finds (count pass)
+  DBuf segcache;              // the first segments of each leaf's list (count pass)
   DBuf iperm;                 // int32 [n]: target order inside each listed leaf
 };
 

@@ -11,10 +11,8 @@
 //   * takes a not-accepted leaf's particles,
 //   * pushes the children of a not-accepted internal node whose L-infinity
 //     gap to the target leaf is <= fsrrmax,
-// and finally appends the leaf's own particles.  One thread walks one
-// (leaf, ancestor sibling) subtree (two passes: count, then fill), with its
-// LIFO stack in HBM laid out level-major so the threads of a wave touch
-// neighbouring words.
+// and finally appends the leaf's own particles.  One wave walks one leaf's
+// list, up to 64 nodes of its LIFO stack (in LDS) at a time.
 //
 // Compiled with -ffp-contract=off so dist2, l2, dtt2 and the corner
 // diagonals round exactly as the reference's x86 float code does.
@@ -31,12 +29,12 @@ namespace {
 struct ListParams {
   float fsrrmax, fsrrmax2, tan_oa;
   int tdpts;                 // pseudo-particles per node (1 or 12)
-  int64_t stack_depth;
-  int64_t nthreads;
+  int stack_cap;             // nodes the wave's LDS stack holds
+  int stack_reserve;         // of which the last ones are for one-by-one walking
   int64_t *overflow;
-  // the count pass keeps each walk's first `cache` segments (offset or node
-  // id, count or -1) at cache_seg[i * nthreads + walk]; the fill pass copies
-  // the walks that fit instead of walking them again
+  // the count pass keeps each leaf's first `cache` segments (offset or node
+  // id, count or -1) at cache_seg[leaf * cache + i]; only longer lists are
+  // walked again to be filled in
   int cache;
   int2 *cache_seg;
 };
@@ -86,283 +84,261 @@ __global__ void k_slot_box(int64_t nboxes, const int64_t *leaf_base,
     slot_box[k] = (int32_t)b;
 }
 
-// The walk of one leaf is a concatenation of independent walks.  Popping an
-// ancestor of the leaf pushes its children except the leaf (left, then
-// right), so below the ancestor at depth d - 1 the LIFO finishes the right
-// child's subtree before the left one's: the list is the walks of the
-// siblings of the leaf's ancestors (the other child at each depth d), right
-// siblings in increasing d, then left siblings in decreasing d, then the
-// leaf's own particles.  One thread walks one (leaf, d) sibling subtree.
-// Returns the sibling at depth d (-1 if none) and whether it is the right
-// child.
-__device__ __forceinline__ int64_t ancestor_sibling(const hsr_node *__restrict__ t, int64_t root,
-                                                    int64_t tl, int64_t toff, int64_t tend, int d,
-                                                    bool *right) {
-  int64_t a = root;
-  int64_t sib = -1;
-  *right = true;
-  // a leaf that is the root is no ancestor of itself: its walk starts at
-  // the root like any other (RCBForceTree.cxx:936-962) and takes the root's
-  // particles before the own ones are appended
-  if (root == tl) return d == 1 ? root : -1;
-  for (int i = 1; i <= d; ++i) {
-    if (a == tl) return -1;
-    const hsr_node &A = t[a];
-    const int64_t cl = A.cl, cr = A.cr;
-    const bool in_l = cl > 0 && t[cl].count > 0 && t[cl].offset <= toff &&
-                      tend <= t[cl].offset + t[cl].count;
-    if (in_l) {
-      sib = cr;
-      *right = true;
-      a = cl;
-    } else {
-      if (cr <= 0) return -1;
-      sib = cl;
-      *right = false;
-      a = cr;
+// What a stack slot of the walk holds: a node still to be looked at (a node
+// reached from a not-accepted one must first pass the distance test; an
+// ancestor's child need not) or a decided segment, waiting for those that
+// come before it in the list.
+enum { W_NODE = 0, W_NODE_GAP = 1, W_RANGE = 2, W_PSEUDO = 3 };
+
+// Whether node N, seen from leaf L's centre, is too large to be accepted
+// (RCBForceTree.cxx:975-1030: the shortest edge, then the four space
+// diagonals with z fixed min to max, against dist2 tan^2 oa).
+__device__ __forceinline__ bool looks_big(const hsr_node &N, const float *lxc, float dist2,
+                                          float tanOA) {
+  const float sx = N.xmax[0] - N.xmin[0];
+  const float sy = N.xmax[1] - N.xmin[1];
+  const float sz = N.xmax[2] - N.xmin[2];
+  const float sx2 = sx * sx, sy2 = sy * sy, sz2 = sz * sz;
+  const float syz = (sz2 < sy2) ? sz2 : sy2;
+  const float l2 = (syz < sx2) ? syz : sx2;
+  const float dtt2 = dist2 * tanOA * tanOA;
+  bool big = l2 > dtt2;
+  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j) {
+      const float x1 = (i == 0 ? N.xmin[0] : N.xmax[0]) - lxc[0];
+      const float y1 = (j == 0 ? N.xmin[1] : N.xmax[1]) - lxc[1];
+      const float z1 = N.xmin[2] - lxc[2];
+      const float x2 = (i == 0 ? N.xmax[0] : N.xmin[0]) - lxc[0];
+      const float y2 = (j == 0 ? N.xmax[1] : N.xmin[1]) - lxc[1];
+      const float z2 = N.xmax[2] - lxc[2];
+      const float ddx = x1 - x2, ddy = y1 - y2, ddz = z1 - z2;
+      const float dh2 = ddx * ddx + ddy * ddy + ddz * ddz;
+      big = big || dh2 > dtt2;
     }
-  }
-  if (sib <= 0 || t[sib].count <= 0) return -1;
-  return sib;
+  return big;
 }
 
+// The list of one leaf by one wave.  The reference walks a LIFO one node at a
+// time; what becomes of a node depends on the node and the leaf alone, so a
+// wave takes the top 64 slots at once, decides all of them, puts the children
+// of the opened nodes in their parent's place (right child on top, as the
+// LIFO pops it first) and emits the segments above the first opened node --
+// everything below it has to wait for that node's subtree and goes back on
+// the stack, decided.  The segments come out in the LIFO's order, and the
+// number of rounds is about the depth of the tree plus a 64th of the nodes
+// looked at, each round one dependent node load, where one thread per walk
+// took a round per node and the longest walk set the time (latency-bound
+// still, but with every lane of a round in flight).  Count pass, before and
+// now: 1.35 and 0.055 ms at 48^3 clustered with leaves of 128, 1.38 and 0.35
+// ms at 256^3 with leaves of 512; the list phase 4.45 and 2.59 ms there.
+//
+// A round replaces k slots by at most 2 k, so the stack could grow by 64 a
+// round; when fewer than stack_reserve slots are free above it, the wave
+// walks one node at a time, whose height grows by at most one per level of
+// the tree (stack_reserve covers the tree's depth).
 template <bool FILL>
 __global__ void __launch_bounds__(64)
 k_walk(const hsr_node *__restrict__ t, const int32_t *__restrict__ leaves,
-       const int32_t *__restrict__ leaf_box, const int64_t *__restrict__ cbase,
-       int64_t nleaves, int ndepth, ListParams lp, int32_t *stack, int64_t *nseg_out,
-       int64_t *nent_out, uint8_t *side_out, const int64_t *seg_ptr, const int64_t *slot_seg,
-       const int64_t *slot_ent, int64_t *seg_a, int64_t *seg_b, int64_t *seg_e) {
-  const int64_t gid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (gid >= nleaves * ndepth) return;
-  const int64_t k = gid / ndepth;
-  const int d = (int)(gid - k * ndepth) + 1;
-  const int64_t tl = leaves[k];
-  const int64_t root = cbase[leaf_box[k]];
-  const float fsrrmax = lp.fsrrmax, fsrrmax2 = lp.fsrrmax2;
-  const float tanOA = lp.tan_oa;
+       const int32_t *__restrict__ leaf_box, const int64_t *__restrict__ cbase, int64_t nleaves,
+       ListParams lp, int64_t *nseg_out, int64_t *nent_out, const int64_t *seg_ptr,
+       int64_t *seg_a, int64_t *seg_b) {
+  extern __shared__ int32_t stk[];
+  uint8_t *kind = reinterpret_cast<uint8_t *>(stk + lp.stack_cap);
+  const int64_t k = blockIdx.x;
+  if (k >= nleaves) return;
+  // fill pass: only the lists the cache does not hold whole
+  if (FILL && nseg_out[k] - 1 <= lp.cache) return;
+  const int l = lane_id();
+  const int32_t tl = leaves[k];
+  const int32_t root = (int32_t)cbase[leaf_box[k]];
   const hsr_node &L = t[tl];
   const int64_t toff = L.offset, tend = L.offset + L.count;
-  if (FILL && nseg_out[gid] <= lp.cache) {
-    // the count pass kept this walk's segments: copy them
-    const int64_t ns = nseg_out[gid];
-    const int64_t so = seg_ptr[k] + slot_seg[gid];
-    int64_t nent = slot_ent[gid];
-    for (int64_t i = 0; i < ns; ++i) {
-      const int2 s = lp.cache_seg[i * lp.nthreads + gid];
-      seg_a[so + i] = s.x;
-      seg_b[so + i] = s.y;
-      seg_e[so + i] = nent;
-      nent += s.y < 0 ? lp.tdpts : s.y;
-    }
-    return;
+  const float lxc[3] = {L.xc[0], L.xc[1], L.xc[2]};
+  const float lmin[3] = {L.xmin[0], L.xmin[1], L.xmin[2]};
+  const float lmax[3] = {L.xmax[0], L.xmax[1], L.xmax[2]};
+  const int64_t so = FILL ? seg_ptr[k] : 0;
+  int64_t nseg = 0;   // emitted so far (uniform)
+  int64_t nent = 0;   // this lane's share of their entries
+  int h = 1;          // stack height (uniform)
+  if (l == 0) {
+    stk[0] = root;
+    kind[0] = W_NODE;
   }
-  bool right;
-  const int64_t sib = ancestor_sibling(t, root, tl, toff, tend, d, &right);
-  if (!FILL) side_out[gid] = right ? 1 : 0;
-  if (sib < 0) {
-    if (!FILL) {
-      nseg_out[gid] = 0;
-      nent_out[gid] = 0;
+  __syncthreads();
+  while (h > 0) {
+    const int room = lp.stack_cap - h - lp.stack_reserve;
+    const int b = room > 0 ? min(min(64, h), room) : 1;
+    if (h >= lp.stack_cap) {  // unreachable while the reserve covers the depth
+      if (l == 0) atomicAdd((unsigned long long *)lp.overflow, 1ull);
+      break;
     }
-    return;
-  }
-  const float lxc0 = L.xc[0], lxc1 = L.xc[1], lxc2 = L.xc[2];
-  float lmin[3] = {L.xmin[0], L.xmin[1], L.xmin[2]};
-  float lmax[3] = {L.xmax[0], L.xmax[1], L.xmax[2]};
-  int32_t *stk = stack + gid;
-  const int64_t sstride = lp.nthreads;
-  int64_t sp = 0;
-  int64_t nseg = 0, nent = FILL ? slot_ent[gid] : 0;
-  const int64_t so = FILL ? seg_ptr[k] + slot_seg[gid] : 0;
-  bool dead = false;
-  stk[0] = (int32_t)sib;
-  sp = 1;
-  // the LIFO never holds more than (tree depth + 2) nodes; the guard only
-  // protects the stack buffer
-#define PUSH(v)                                             \
-  do {                                                      \
-    if (sp >= lp.stack_depth) {                             \
-      atomicAdd((unsigned long long *)lp.overflow, 1ull);   \
-      dead = true;                                          \
-    } else {                                                \
-      stk[sp * sstride] = (int32_t)(v);                     \
-      ++sp;                                                 \
-    }                                                       \
-  } while (0)
-#define EMIT(A, B, LEN)                                                        \
-  do {                                                                         \
-    if (FILL) {                                                                \
-      seg_a[so + nseg] = (A);                                                  \
-      seg_b[so + nseg] = (B);                                                  \
-      seg_e[so + nseg] = nent;                                                 \
-    } else if (nseg < lp.cache) {                                              \
-      lp.cache_seg[nseg * lp.nthreads + gid] = make_int2((int)(A), (int)(B));  \
-    }                                                                          \
-    ++nseg;                                                                    \
-    nent += (LEN);                                                             \
-  } while (0)
-  while (sp > 0 && !dead) {
-    --sp;
-    const int64_t tln = stk[sp * sstride];
-    const hsr_node &N = t[tln];
-    if (tln < tl) {
-      // ancestors of tl are exactly the nodes whose particle range contains
-      // tl's (node ranges nest or are disjoint)
-      if (N.offset <= toff && tend <= N.offset + N.count) {
-        const int64_t cr = N.cr, cl = N.cl;
-        if (cl != tl && cl > 0 && t[cl].count > 0) PUSH(cl);
-        if (cr != tl && cr > 0 && t[cr].count > 0) PUSH(cr);
-        continue;
-      }
-    }
-    float dx = N.xc[0] - lxc0;
-    float dy = N.xc[1] - lxc1;
-    float dz = N.xc[2] - lxc2;
-    float dist2 = dx * dx + dy * dy + dz * dz;
-    float sx = N.xmax[0] - N.xmin[0];
-    float sy = N.xmax[1] - N.xmin[1];
-    float sz = N.xmax[2] - N.xmin[2];
-    float sx2 = sx * sx, sy2 = sy * sy, sz2 = sz * sz;
-    float syz = (sz2 < sy2) ? sz2 : sy2;
-    float l2 = (syz < sx2) ? syz : sx2;
-    float dtt2 = dist2 * tanOA * tanOA;
-    bool looksBig;
-    if (l2 > dtt2) {
-      looksBig = true;
-    } else {
-      looksBig = false;
-      for (int i = 0; i < 2 && !looksBig; ++i)
-        for (int j = 0; j < 2; ++j) {
-          float x1 = (i == 0 ? N.xmin[0] : N.xmax[0]) - lxc0;
-          float y1 = (j == 0 ? N.xmin[1] : N.xmax[1]) - lxc1;
-          float z1 = N.xmin[2] - lxc2;
-          float x2 = (i == 0 ? N.xmax[0] : N.xmin[0]) - lxc0;
-          float y2 = (j == 0 ? N.xmax[1] : N.xmin[1]) - lxc1;
-          float z2 = N.xmax[2] - lxc2;
-          float ddx = x1 - x2, ddy = y1 - y2, ddz = z1 - z2;
-          float dh2 = ddx * ddx + ddy * ddy + ddz * ddz;
-          if (dh2 > dtt2) {
-            looksBig = true;
-            break;
+    // this lane's slot, its outcome (the children to push or a segment)
+    int nout = 0, k0 = W_RANGE, k1 = W_RANGE;
+    int32_t v0 = 0, v1 = 0;
+    int64_t sa = 0, sb = 0;
+    if (l < b) {
+      const int32_t id = stk[h - 1 - l];
+      const int kd = kind[h - 1 - l];
+      const hsr_node &N = t[id];
+      const int64_t cnt = N.count, noff = N.offset;
+      const int32_t cl = (int32_t)N.cl, cr = (int32_t)N.cr;
+      v0 = id;
+      if (kd >= W_RANGE) {
+        nout = 1;
+        k0 = kd;
+      } else if (id < tl && noff <= toff && tend <= noff + cnt) {
+        // an ancestor of the leaf: its children but the leaf
+        if (cr > 0 && cr != tl) {
+          v0 = cr;
+          k0 = W_NODE;
+          nout = 1;
+        }
+        if (cl > 0 && cl != tl) {
+          (nout ? v1 : v0) = cl;
+          (nout ? k1 : k0) = W_NODE;
+          ++nout;
+        }
+      } else {
+        bool near = cnt > 0 || id == root;  // the root of an empty box is looked at
+        if (kd == W_NODE_GAP) {
+          for (int i = 0; i < 3; ++i) {
+            float dist = 0;
+            if (lmax[i] < N.xmin[i]) dist = N.xmin[i] - lmax[i];
+            else if (lmin[i] > N.xmax[i]) dist = lmin[i] - N.xmax[i];
+            if (dist > lp.fsrrmax) near = false;
           }
         }
-    }
-    if (!looksBig) {
-      if (dist2 > fsrrmax2) continue;
-      if (N.count <= lp.tdpts) {
-        EMIT(N.offset, N.count, N.count);
-        continue;
-      }
-      EMIT(tln, -1, lp.tdpts);
-      continue;
-    } else if (N.cr == 0 && N.cl == 0) {
-      EMIT(N.offset, N.count, N.count);
-      continue;
-    }
-    const int64_t ch[2] = {N.cl, N.cr};
-    for (int q = 0; q < 2; ++q) {
-      const int64_t c = ch[q];
-      if (c > 0 && t[c].count > 0) {
-        const hsr_node &Cn = t[c];
-        bool close = true;
-        for (int i = 0; i < 3; ++i) {
-          float dist = 0;
-          if (lmax[i] < Cn.xmin[i]) dist = Cn.xmin[i] - lmax[i];
-          else if (lmin[i] > Cn.xmax[i]) dist = lmin[i] - Cn.xmax[i];
-          if (dist > fsrrmax) {
-            close = false;
-            break;
+        if (near) {
+          const float dx = N.xc[0] - lxc[0];
+          const float dy = N.xc[1] - lxc[1];
+          const float dz = N.xc[2] - lxc[2];
+          const float dist2 = dx * dx + dy * dy + dz * dz;
+          if (!looks_big(N, lxc, dist2, lp.tan_oa)) {
+            if (!(dist2 > lp.fsrrmax2)) {
+              nout = 1;
+              k0 = cnt <= lp.tdpts ? W_RANGE : W_PSEUDO;
+            }
+          } else if (cr == 0 && cl == 0) {
+            nout = 1;
+            k0 = W_RANGE;
+          } else {
+            if (cr > 0) {
+              v0 = cr;
+              k0 = W_NODE_GAP;
+              nout = 1;
+            }
+            if (cl > 0) {
+              (nout ? v1 : v0) = cl;
+              (nout ? k1 : k0) = W_NODE_GAP;
+              ++nout;
+            }
           }
         }
-        if (close) PUSH(c);
+      }
+      sa = k0 == W_PSEUDO ? (int64_t)id : noff;
+      sb = k0 == W_PSEUDO ? -1 : cnt;
+    }
+    // the lanes before the first one that opened a node are done
+    const uint64_t opened = __ballot(nout > 0 && k0 < W_RANGE);
+    const int first = opened ? (int)__builtin_ctzll(opened) : 64;
+    const bool emit = l < first && nout == 1;
+    const uint64_t em = __ballot(emit);
+    if (emit) {
+      const int64_t s = nseg + __popcll(em & lanemask_lt());
+      if (FILL) {
+        seg_a[so + s] = sa;
+        seg_b[so + s] = sb;
+      } else {
+        if (s < lp.cache) lp.cache_seg[k * lp.cache + s] = make_int2((int)sa, (int)sb);
+        nent += sb < 0 ? lp.tdpts : sb;
       }
     }
+    nseg += __popcll(em);
+    // the rest go back on the stack, the first lane's on top
+    const int np = l >= first ? nout : 0;
+    const uint64_t p1 = __ballot(np >= 1), p2 = __ballot(np == 2);
+    const int total = __popcll(p1) + __popcll(p2);
+    const int before = __popcll(p1 & lanemask_lt()) + __popcll(p2 & lanemask_lt());
+    __syncthreads();  // every slot has been read
+    const int base = h - b + total - 1 - before;
+    if (np >= 1) {
+      stk[base] = v0;
+      kind[base] = (uint8_t)k0;
+    }
+    if (np == 2) {
+      stk[base - 1] = v1;
+      kind[base - 1] = (uint8_t)k1;
+    }
+    h += total - b;
+    __syncthreads();
   }
-#undef PUSH
-#undef EMIT
   if (!FILL) {
-    nseg_out[gid] = nseg;
-    nent_out[gid] = nent;
+    nent = wave_sum_i64(nent);
+    if (l == 0) {
+      nseg_out[k] = nseg + 1;  // and the leaf's own particles
+      nent_out[k] = nent + L.count;
+    }
   }
 }
 
-// Per leaf: the order of its sibling walks (right siblings by increasing
-// depth, left ones by decreasing depth; depths past the leaf's hold empty
-// walks), their segment and entry offsets in the leaf's list, and the
-// leaf's totals with its own particles as the last segment.
-__global__ void k_walk_order(const hsr_node *__restrict__ t, const int32_t *__restrict__ leaves,
-                             int64_t nleaves, int ndepth, const int64_t *cnt_seg,
-                             const int64_t *cnt_ent, const uint8_t *side, int64_t *slot_seg,
-                             int64_t *slot_ent, int64_t *nseg, int64_t *nent) {
-  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= nleaves) return;
-  const int64_t base = k * ndepth;
-  int64_t so = 0, eo = 0;
-  for (int i = 0; i < ndepth; ++i)
-    if (side[base + i]) {
-      slot_seg[base + i] = so;
-      slot_ent[base + i] = eo;
-      so += cnt_seg[base + i];
-      eo += cnt_ent[base + i];
-    }
-  for (int i = ndepth - 1; i >= 0; --i)
-    if (!side[base + i]) {
-      slot_seg[base + i] = so;
-      slot_ent[base + i] = eo;
-      so += cnt_seg[base + i];
-      eo += cnt_ent[base + i];
-    }
-  nseg[k] = so + 1;  // the leaf's own particles
-  nent[k] = eo + t[leaves[k]].count;
-}
-
-__global__ void k_walk_own(const hsr_node *__restrict__ t, const int32_t *__restrict__ leaves,
-                           int64_t nleaves, const int64_t *seg_ptr, const int64_t *ent_ptr,
-                           int64_t *seg_a, int64_t *seg_b, int64_t *seg_e) {
-  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= nleaves) return;
-  const hsr_node &L = t[leaves[k]];
-  const int64_t s = seg_ptr[k + 1] - 1;
-  seg_a[s] = L.offset;
-  seg_b[s] = L.count;
-  seg_e[s] = ent_ptr[k + 1] - ent_ptr[k] - L.count;
-}
-
-// Expand segments into j indices (one wave per listed leaf): particle
-// ranges by all lanes, the T pseudo-particles of node a as indices
-// count + T a + j (RCBForceTree.cxx:1051-1060).
+// The segments of every listed leaf in place, with their entry offsets, and
+// expanded into j indices (one wave per leaf): particle ranges by all lanes,
+// the T pseudo-particles of node a as indices count + T a + j
+// (RCBForceTree.cxx:1051-1060).  The segments come from the count pass's
+// cache, or for the lists it does not hold whole from where the second walk
+// left them; the leaf's own particles are the last segment.
 __global__ void __launch_bounds__(64)
-k_expand(int64_t nleaves, int64_t n, int tdpts, const int64_t *__restrict__ seg_ptr,
-         const int64_t *__restrict__ seg_a, const int64_t *__restrict__ seg_b,
+k_expand(int64_t nleaves, int64_t n, ListParams lp, const hsr_node *__restrict__ t,
+         const int32_t *__restrict__ leaves, const int64_t *__restrict__ seg_ptr,
+         int64_t *__restrict__ seg_a, int64_t *__restrict__ seg_b, int64_t *__restrict__ seg_e,
          const int64_t *__restrict__ ent_ptr, int32_t *__restrict__ jidx) {
-  int64_t k = blockIdx.x;
+  const int64_t k = blockIdx.x;
   if (k >= nleaves) return;
-  int l = lane_id();
-  int64_t e = ent_ptr[k];
+  const int l = lane_id();
+  const int tdpts = lp.tdpts;
+  const int64_t e0 = ent_ptr[k];
   const int64_t s0 = seg_ptr[k], s1 = seg_ptr[k + 1];
+  const bool cached = s1 - s0 - 1 <= lp.cache;
+  int64_t e = 0;
   // 64 segments at a time: lane i reads segment s + i, a wave prefix of
   // their entry counts places them, then they are written one by one
   for (int64_t s = s0; s < s1; s += 64) {
-    const bool v = s + l < s1;
-    const int64_t a = v ? seg_a[s + l] : 0, b = v ? seg_b[s + l] : 0;
-    const int64_t len = !v ? 0 : (b < 0 ? (int64_t)tdpts : b);
+    const int64_t sl = s + l;
+    int64_t a = 0, b = 0;
+    if (sl == s1 - 1) {
+      const hsr_node &L = t[leaves[k]];
+      a = L.offset;
+      b = L.count;
+    } else if (sl < s1 && cached) {
+      const int2 q = lp.cache_seg[k * lp.cache + (sl - s0)];
+      a = q.x;
+      b = q.y;
+    } else if (sl < s1) {
+      a = seg_a[sl];
+      b = seg_b[sl];
+    }
+    const int64_t len = b < 0 ? (int64_t)tdpts : b;
     int64_t inc = len;  // inclusive prefix over the lanes
     for (int o = 1; o < 64; o <<= 1) {
       const int64_t y = (int64_t)__shfl_up((long long)inc, o);
       if (l >= o) inc += y;
     }
+    if (sl < s1) {
+      seg_a[sl] = a;
+      seg_b[sl] = b;
+      seg_e[sl] = e + inc - len;
+    }
     const int m = (int)min<int64_t>(64, s1 - s);
     for (int j = 0; j < m; ++j) {
-      const int64_t aj = (int64_t)__shfl((long long)a, j), bj = (int64_t)__shfl((long long)b, j);
-      const int64_t ej = e + (int64_t)__shfl((long long)(inc - len), j);
+      const int32_t aj = readlane_i32((int32_t)a, j), bj = readlane_i32((int32_t)b, j);
+      int32_t *out = jidx + e0 + e + (int64_t)readlane_u64((uint64_t)(inc - len), j);
       if (bj < 0) {
-        if (l < tdpts) jidx[ej + l] = (int32_t)(n + tdpts * aj + l);
+        if (l < tdpts) out[l] = (int32_t)(n + (int64_t)tdpts * aj + l);
       } else {
-        for (int64_t i = l; i < bj; i += 64) jidx[ej + i] = (int32_t)(aj + i);
+        for (int i = l; i < bj; i += 64) out[i] = aj + i;
       }
     }
-    e += (int64_t)__shfl((long long)inc, 63);
+    e += (int64_t)readlane_u64((uint64_t)inc, 63);
   }
 }
 
@@ -457,39 +433,26 @@ hsr_status lists_build_device(hsr_ctx *c, const float *min_force_h,
   HSR_HIP(dbuf_reserve(S.h, sizeof(int64_t) * 2 * (nl + 1) + 64));
   int64_t *nseg = dptr<int64_t>(S.h);
   int64_t *nent = nseg + nl + 1;
-  const int64_t depth = T.max_depth + 8;
-  // one walk per (leaf, ancestor sibling at depth 1 .. max_depth)
-  const int ndepth = (int)std::max<int64_t>(1, T.max_depth);
-  const int64_t nwalk = std::max<int64_t>(1, nl) * ndepth;
-  HSR_HIP(dbuf_reserve(LS.stack, sizeof(int32_t) * (size_t)nwalk * depth));
-  HSR_HIP(dbuf_reserve(LS.walk, (sizeof(int64_t) * 4 + 1) * (size_t)nwalk + 64));
-  int64_t *cnt_seg = dptr<int64_t>(LS.walk);
-  int64_t *cnt_ent = cnt_seg + nwalk;
-  int64_t *slot_seg = cnt_ent + nwalk;
-  int64_t *slot_ent = slot_seg + nwalk;
-  uint8_t *side = reinterpret_cast<uint8_t *>(slot_ent + nwalk);
   ListParams lp;
   lp.fsrrmax = c->p.fsrrmax;
   lp.fsrrmax2 = c->p.fsrrmax * c->p.fsrrmax;
   lp.tan_oa = c->p.tan_oa;
   lp.tdpts = c->p.tdpts;
-  lp.stack_depth = depth;
-  lp.nthreads = nwalk;
-  // segment cache: up to 128 per walk within 2 GiB (at 256^3, 1.1 GB)
-  lp.cache = (int)std::min<int64_t>(128, ((int64_t)1 << 31) / ((int64_t)sizeof(int2) * nwalk));
-  HSR_HIP(dbuf_reserve(LS.segcache, sizeof(int2) * (size_t)std::max(lp.cache, 1) * (size_t)nwalk));
+  // 1024 slots beside the reserve: 5.2 KB of LDS a wave
+  lp.stack_reserve = (int)std::min<int64_t>(T.max_depth + 4, 8192);
+  lp.stack_cap = 1024 + lp.stack_reserve;
+  const size_t lds = ((sizeof(int32_t) + 1) * (size_t)lp.stack_cap + 15) / 16 * 16;
+  // segment cache: up to 512 per leaf within 2 GiB (at 256^3, 0.2 GB)
+  lp.cache = (int)std::min<int64_t>(512, ((int64_t)1 << 31) / ((int64_t)sizeof(int2) * std::max<int64_t>(1, nl)));
+  HSR_HIP(dbuf_reserve(LS.segcache, sizeof(int2) * (size_t)std::max(lp.cache, 1) * (size_t)std::max<int64_t>(1, nl)));
   lp.cache_seg = dptr<int2>(LS.segcache);
   HSR_HIP(dbuf_reserve(S.counters, 256));
   lp.overflow = dptr<int64_t>(S.counters) + 20;
   k_zero_i64<<<1, 64, 0, st>>>(lp.overflow, 1);
   const hsr_node *cn = dptr<hsr_node>(T.canon_nodes);
-  int32_t *stk = dptr<int32_t>(LS.stack);
   if (nl > 0) {
-    k_walk<false><<<nblk(nl * ndepth, 64), 64, 0, st>>>(cn, leaves, leaf_box, d_cbase, nl, ndepth, lp,
-                                                          stk, cnt_seg, cnt_ent, side, nullptr, nullptr,
-                                                          nullptr, nullptr, nullptr, nullptr);
-    k_walk_order<<<nblk(nl, 64), 64, 0, st>>>(cn, leaves, nl, ndepth, cnt_seg, cnt_ent, side,
-                                              slot_seg, slot_ent, nseg, nent);
+    k_walk<false><<<(unsigned)nl, 64, lds, st>>>(cn, leaves, leaf_box, d_cbase, nl, lp, nseg, nent,
+                                                 nullptr, nullptr, nullptr);
     k_zero_i64<<<1, 64, 0, st>>>(nseg + nl, 1);
     k_zero_i64<<<1, 64, 0, st>>>(nent + nl, 1);
     if (excl_scan(c, nseg, dptr<int64_t>(LS.seg_ptr), nl + 1) != HSR_OK) return HSR_ERR_HIP;
@@ -510,14 +473,10 @@ hsr_status lists_build_device(hsr_ctx *c, const float *min_force_h,
   int64_t *seg_e = seg_b + LS.nsegs + 1;
   HSR_HIP(dbuf_reserve(LS.jidx, sizeof(int32_t) * (LS.nentries + 1)));
   if (nl > 0) {
-    k_walk<true><<<nblk(nl * ndepth, 64), 64, 0, st>>>(cn, leaves, leaf_box, d_cbase, nl, ndepth, lp,
-                                                         stk, cnt_seg, nullptr, nullptr,
-                                                         dptr<int64_t>(LS.seg_ptr),
-                                                         slot_seg, slot_ent, seg_a, seg_b, seg_e);
-    k_walk_own<<<nblk(nl, 64), 64, 0, st>>>(cn, leaves, nl, dptr<int64_t>(LS.seg_ptr),
-                                            dptr<int64_t>(LS.ent_ptr), seg_a, seg_b, seg_e);
-    k_expand<<<(unsigned)nl, 64, 0, st>>>(nl, n, c->p.tdpts, dptr<int64_t>(LS.seg_ptr), seg_a, seg_b,
-                                          dptr<int64_t>(LS.ent_ptr), dptr<int32_t>(LS.jidx));
+    k_walk<true><<<(unsigned)nl, 64, lds, st>>>(cn, leaves, leaf_box, d_cbase, nl, lp, nseg, nullptr,
+                                                dptr<int64_t>(LS.seg_ptr), seg_a, seg_b);
+    k_expand<<<(unsigned)nl, 64, 0, st>>>(nl, n, lp, cn, leaves, dptr<int64_t>(LS.seg_ptr), seg_a, seg_b,
+                                          seg_e, dptr<int64_t>(LS.ent_ptr), dptr<int32_t>(LS.jidx));
   }
   // pairs = sum count * list length
   int64_t *d_pairs = dptr<int64_t>(S.counters) + 16;
