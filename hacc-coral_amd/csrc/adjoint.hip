@@ -27,6 +27,7 @@
 //                 hold the leaf); pseudo pass per (target leaf, pseudo
 //                 segment).  Used when W does not fit in device memory.
 #include "hsr_internal.h"
+#include "queue.h"
 #include "wave.h"
 
 #include <hipcub/hipcub.hpp>
@@ -137,10 +138,10 @@ k_adj(const hsr_node *__restrict__ cn, const AItem *__restrict__ items,
   float (*red)[64 * R] = reinterpret_cast<float (*)[64 * R]>(&tA[0]);
   const int l = lane_id();
   const int64_t nitems = *nitems_p;
+  __shared__ QueueState qs;
+  queue_begin(&qs);
   for (;;) {
-    int64_t it = 0;
-    if (l == 0) it = (int64_t)atomicAdd(qctr, 1ull);
-    it = (int64_t)readlane_u64((uint64_t)it, 0);
+    const int64_t it = queue_pop(qctr, nitems, &qs);
     if (it >= nitems) break;
     const AItem I = items[it];
     const hsr_node &nd = cn[I.leaf];
@@ -454,10 +455,10 @@ adj_fused_body(const hsr_node *__restrict__ cn, const AItem *__restrict__ items,
   float (*red)[64 * FR] = reinterpret_cast<float (*)[64 * FR]>(&tile[0]);
   const int l = lane_id();
   const int64_t nitems = *nitems_p;
+  __shared__ QueueState qs;
+  queue_begin(&qs);
   for (;;) {
-    int64_t it = 0;
-    if (l == 0) it = (int64_t)atomicAdd(qctr, 1ull);
-    it = (int64_t)readlane_u64((uint64_t)it, 0);
+    const int64_t it = queue_pop(qctr, nitems, &qs);
     if (it >= nitems) break;
     const AItem I = items[it];
     const hsr_node &nd = cn[I.leaf];
@@ -908,8 +909,8 @@ __global__ void k_fill(int64_t n, float *a) {
   if (k < n) a[k] = 0.f;
 }
 
-__global__ void k_zero_u64a(unsigned long long *p) {
-  if (threadIdx.x == 0) *p = 0ull;
+__global__ void k_queue_reset(unsigned long long *q, int64_t grid) {
+  queue_reset(q, (int)threadIdx.x, grid);
 }
 
 // Canonical parent of every node.
@@ -1102,7 +1103,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   HSR_HIP(hipStreamSynchronize(st));
   HSR_HIP(hipGetLastError());
   // buffers of the passes (reserved here so that a captured graph allocates nothing)
-  HSR_HIP(dbuf_reserve(A.qctr, 64));
+  HSR_HIP(dbuf_reserve(A.qctr, sizeof(unsigned long long) * QWORDS));
   HSR_HIP(dbuf_reserve(A.part, sizeof(float) * (std::max(A.fw_part, A.tr_part) + 1)));
   HSR_HIP(dbuf_reserve(A.H, sizeof(float) * 3 * (nn + 1) + sizeof(float) * 3 * (A.npseudo + 1)));
   A.gen = c->lists_gen;
@@ -1199,8 +1200,8 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
   }
   // target pass
   if (A.n_fw_items) {
-    k_zero_u64a<<<1, 64, 0, st>>>(q);
-    const int64_t grid = std::min<int64_t>(A.n_fw_items, (int64_t)std::max(1, c->num_cus) * wpc);
+    const int64_t grid = (int64_t)std::max(1, c->num_cus) * wpc;
+    k_queue_reset<<<1, 64, 0, st>>>(q, grid);
 #define LA(MODE, ORD, ITEMS, CNT)                                                          \
   k_adj<MODE, ORD><<<(unsigned)grid, 64, 0, st>>>(cn, ITEMS, CNT, MODE == 0 ?               \
       dptr<int32_t>(c->lists.jidx) : dptr<int32_t>(A.tj), pj, lx, ly, lz, L, q, gx, gy, gz, part)
@@ -1236,8 +1237,8 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
                                                   seg_e, cn, pj, W, W + ne, W + 2 * ne, gx, gy, gz);
   // source pass of the two-pass schedule
   if (!A.fused && A.n_tr_items) {
-    k_zero_u64a<<<1, 64, 0, st>>>(q);
-    const int64_t grid = std::min<int64_t>(A.n_tr_items, (int64_t)std::max(1, c->num_cus) * wpc);
+    const int64_t grid = (int64_t)std::max(1, c->num_cus) * wpc;
+    k_queue_reset<<<1, 64, 0, st>>>(q, grid);
     if (L.order == 6) LA(1, 6, dptr<AItem>(A.tr_items), counts + 1);
     else LA(1, 5, dptr<AItem>(A.tr_items), counts + 1);
 #undef LA

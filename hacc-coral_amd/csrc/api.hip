@@ -616,15 +616,13 @@ hsr_status hsr_lists_many(hsr_ctx *c, const float *min_force,
   return HSR_OK;
 }
 
-// Pairs the last force phase evaluated (its kernel's counter, qctr[1]).
+// Pairs the last force phase evaluated, and of those the unmasked ones (the
+// totals behind its work queue).
 static hipError_t read_evaluated(hsr_ctx *c) {
-  c->evaluated_pairs = c->unmasked_pairs = 0;
+  c->pair_counts[0] = c->pair_counts[1] = 0;
   if (c->lists.nleaves == 0 || c->lists.nitems == 0 || !c->s.qctr.p) return hipSuccess;
-  hipError_t e = hipMemcpyAsync(&c->evaluated_pairs, dptr<unsigned long long>(c->s.qctr) + 1,
-                                sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
-  if (e != hipSuccess) return e;
-  return hipMemcpyAsync(&c->unmasked_pairs, dptr<unsigned long long>(c->s.qctr) + 2,
-                        sizeof(int64_t), hipMemcpyDeviceToHost, c->stream);
+  return hipMemcpyAsync(c->pair_counts, dptr<unsigned long long>(c->s.qctr) + FORCE_TOTALS,
+                        sizeof(c->pair_counts), hipMemcpyDeviceToHost, c->stream);
 }
 
 hsr_status hsr_forces(hsr_ctx *c, float *ax, float *ay, float *az,
@@ -881,8 +879,8 @@ hsr_status hsr_get_stats(hsr_ctx *c, hsr_stats *st) {
   st->segments = c->lists.nsegs;
   st->entries = c->lists.nentries;
   st->pairs = c->lists.pairs;
-  st->evaluated_pairs = c->evaluated_pairs;
-  st->unmasked_pairs = c->unmasked_pairs;
+  st->evaluated_pairs = c->pair_counts[0];
+  st->unmasked_pairs = c->pair_counts[1];
   st->graph_captures = c->graph_captures;
   st->graph_replays = c->graph_launches - c->graph_captures;
   st->build_ms = c->build_ms;

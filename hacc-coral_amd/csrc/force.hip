@@ -18,6 +18,7 @@
 // reads fall in distinct banks).  Chunk partials of long lists are summed in
 // chunk order afterwards, so results are bitwise reproducible.
 #include "hsr_internal.h"
+#include "queue.h"
 #include "wave.h"
 
 #include <hipcub/hipcub.hpp>
@@ -54,7 +55,7 @@ constexpr int lds_entries() {
 
 struct Item {
   int32_t leaf;     // listed-leaf index
-  int32_t chunk;    // chunk index within the leaf's list
+  int32_t cls;      // work class (0 = heaviest)
   int64_t e0, e1;   // list entry range
   int64_t pbase;    // partial-force offset (-1: write F directly)
 };
@@ -229,19 +230,19 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
   const int l = lane_id();
   const int64_t nitems = *nitems_p;
   const float c0 = L.c[0], rcs = L.rcs;
+  __shared__ QueueState qs;
+  queue_begin(&qs);
   for (;;) {
-    int64_t it = 0;
-    if (l == 0) it = (int64_t)atomicAdd(qctr, 1ull);
-    it = (int64_t)readlane_u64((uint64_t)it, 0);
+    const int64_t it = queue_pop(qctr, nitems, &qs);
     if (it >= nitems) break;
     const Item I = items[it];
     const hsr_node &nd = cn[leaves[I.leaf]];
     const int64_t off = nd.offset, cnt = nd.count;
+    int64_t ev = 0;   // pairs evaluated for this item (culled entries excluded)
+    int64_t evu = 0;  // of which unmasked
     // padding entries: far enough to be masked, near enough to keep every
     // intermediate finite
     const float4 pad = make_float4(nd.xc[0] + 1000.f, nd.xc[1], nd.xc[2], 0.f);
-    int64_t ev = 0;   // pairs evaluated for this item (culled entries excluded)
-    int64_t evu = 0;  // of which unmasked
     // passes over the targets in power-of-two chunks (128, 64, ..., 8, rest)
     // so that every pass fills its groups of lpg = chunk / R lanes
     for (int64_t ib = 0, nib = 0; ib < cnt; ib += nib) {
@@ -409,20 +410,43 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
         }
       }
     }
-    if (l == 0 && ev > 0) atomicAdd(evals, (unsigned long long)ev);
-    if (l == 0 && evu > 0) atomicAdd(evals + 1, (unsigned long long)evu);
+    // into the wave's own slots, summed by k_reduce_chunks: atomics of all
+    // waves on one address would pass one at a time; here nothing waits
+    if (l == 0) {
+      atomicAdd(evals + 2 * (int64_t)blockIdx.x, (unsigned long long)ev);
+      atomicAdd(evals + 2 * (int64_t)blockIdx.x + 1, (unsigned long long)evu);
+    }
   }
 }
 
-// Sum the chunk partials of long lists in chunk order.
+// Sum the chunk partials of long lists in chunk order; the last workgroup
+// sums the waves' pair counts (the waves past the items counted none).
 __global__ void __launch_bounds__(64)
 k_reduce_chunks(const hsr_node *cn, const int32_t *leaves,
                 const int64_t *multi, const int64_t *nmulti_p,
                 const int64_t *leaf_pbase, const int32_t *leaf_nchunk,
-                const int32_t *iperm, const float *part, float *fx, float *fy, float *fz) {
+                const int32_t *iperm, const float *part, float *fx, float *fy, float *fz,
+                const int64_t *nitems_p, int64_t nwaves, const unsigned long long *evals,
+                unsigned long long *totals) {
+  if (blockIdx.x == gridDim.x - 1) {
+    const int64_t nw = min(nwaves, *nitems_p);
+    uint64_t a = 0, b = 0;
+#pragma unroll 8
+    for (int64_t w = threadIdx.x; w < nw; w += 64) {
+      a += evals[2 * w];
+      b += evals[2 * w + 1];
+    }
+    a = wave_sum_u64(a);
+    b = wave_sum_u64(b);
+    if (threadIdx.x == 0) {
+      totals[0] = a;
+      totals[1] = b;
+    }
+    return;
+  }
   // a fixed grid over the device-resident count, so a captured force phase
   // serves every list build
-  for (int64_t k = blockIdx.x; k < *nmulti_p; k += gridDim.x) {
+  for (int64_t k = blockIdx.x; k < *nmulti_p; k += gridDim.x - 1) {
     const int64_t lf = multi[k];
     const hsr_node &nd = cn[leaves[lf]];
     const int64_t cnt = nd.count, off = nd.offset;
@@ -459,48 +483,92 @@ __global__ void k_item_count(int64_t nleaves, const int64_t *ent_ptr,
   psize[k] = c > 1 ? c * 3 * cn[leaves[k]].count : 0;
 }
 
-__global__ void k_item_fill(int64_t nleaves, const int64_t *ent_ptr,
-                            int64_t chunk, const int32_t *nchunk,
-                            const int64_t *item_base, const int64_t *pbase,
-                            const hsr_node *cn, const int32_t *leaves,
-                            Item *items, uint64_t *keys, int32_t *vals,
-                            int64_t *multi, const int64_t *multi_pos,
-                            const int64_t *multi_flag) {
-  int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= nleaves) return;
-  const int64_t e0 = ent_ptr[k], e1 = ent_ptr[k + 1];
-  const int nc = nchunk[k];
-  const int64_t cnt = cn[leaves[k]].count;
-  for (int c = 0; c < nc; ++c) {
-    int64_t j = item_base[k] + c;
-    Item I;
-    I.leaf = (int32_t)k;
-    I.chunk = c;
-    I.e0 = e0 + (int64_t)c * chunk;
-    I.e1 = std::min<int64_t>(e1, I.e0 + chunk);
-    I.pbase = nc > 1 ? pbase[k] + (int64_t)c * 3 * cnt : -1;
-    items[j] = I;
-    // work ~ i-passes * entries
-    uint64_t work = (uint64_t)((cnt + 64 * DEF_R - 1) / (64 * DEF_R)) * (uint64_t)(I.e1 - I.e0);
-    keys[j] = work;
-    vals[j] = (int32_t)j;
+// Work classes of the queue, heaviest first: four to the octave.
+constexpr int NCLASS = 256;
+
+__device__ __forceinline__ int work_class(int64_t targets, int64_t entries) {
+  const int64_t passes = (targets + 64 * DEF_R - 1) / (64 * DEF_R);
+  const float w = (float)(passes * entries + 1);
+  const int b = (int)(__float_as_uint(w) >> 21) - (127 << 2);
+  return NCLASS - 1 - min(NCLASS - 1, b);
+}
+
+__global__ void __launch_bounds__(256)
+k_item_fill(int64_t nleaves, const int64_t *ent_ptr, int64_t chunk, const int32_t *nchunk,
+            const int64_t *item_base, const int64_t *pbase, const hsr_node *cn,
+            const int32_t *leaves, Item *items, uint32_t *hist, int64_t *multi,
+            const int64_t *multi_pos, const int64_t *multi_flag) {
+  __shared__ uint32_t h[NCLASS];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (k < nleaves) {
+    const int64_t e0 = ent_ptr[k], e1 = ent_ptr[k + 1];
+    const int nc = nchunk[k];
+    const int64_t cnt = cn[leaves[k]].count;
+    for (int c = 0; c < nc; ++c) {
+      Item I;
+      I.leaf = (int32_t)k;
+      I.e0 = e0 + (int64_t)c * chunk;
+      I.e1 = std::min<int64_t>(e1, I.e0 + chunk);
+      I.pbase = nc > 1 ? pbase[k] + (int64_t)c * 3 * cnt : -1;
+      I.cls = work_class(cnt, I.e1 - I.e0);
+      items[item_base[k] + c] = I;
+      atomicAdd(&h[I.cls], 1u);
+    }
+    if (multi_flag[k]) multi[multi_pos[k]] = k;
   }
-  if (multi_flag[k]) multi[multi_pos[k]] = k;
+  __syncthreads();
+  if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
 }
 
-__global__ void k_item_permute(int64_t n, const Item *in, const int32_t *order,
-                               Item *out) {
-  int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k < n) out[k] = in[order[k]];
+// The queue in class order: a workgroup reserves its items' slots class by
+// class (hist: items per class; next: slots given out).  The order inside a
+// class, which no result depends on, is whichever workgroup came first.
+__global__ void __launch_bounds__(256)
+k_item_order(int64_t n, const Item *in, const uint32_t *hist, uint32_t *next, Item *out) {
+  __shared__ uint32_t base[NCLASS], cnt[NCLASS];
+  const int t = threadIdx.x;
+  const uint32_t mine = hist[t];
+  base[t] = mine;
+  cnt[t] = 0;
+  __syncthreads();
+  for (int o = 1; o < NCLASS; o <<= 1) {  // inclusive scan
+    const uint32_t v = t >= o ? base[t - o] : 0;
+    __syncthreads();
+    base[t] += v;
+    __syncthreads();
+  }
+  const int64_t k = blockIdx.x * (int64_t)blockDim.x + t;
+  Item I;
+  uint32_t rank = 0;
+  if (k < n) {
+    I = in[k];
+    rank = atomicAdd(&cnt[I.cls], 1u);
+  }
+  __syncthreads();
+  const uint32_t first = base[t] - mine + (cnt[t] ? atomicAdd(&next[t], cnt[t]) : 0u);
+  __syncthreads();
+  base[t] = first;
+  __syncthreads();
+  if (k < n) out[base[I.cls] + rank] = I;
 }
 
-__global__ void k_fill3(int64_t n, float *a, float *b, float *c) {
+// The queue's class counts and slots start from zero.
+__global__ void __launch_bounds__(256) k_zero_classes(uint32_t *hist) {
+  hist[threadIdx.x] = hist[NCLASS + threadIdx.x] = 0;
+}
+
+// Forces and the waves' pair counts start from zero, the work queue from its
+// first items.
+__global__ void k_fill3(int64_t n, float *a, float *b, float *c, unsigned long long *qctr,
+                        int64_t grid) {
   int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (k < n) a[k] = b[k] = c[k] = 0.f;
-}
-
-__global__ void k_zero_u64(unsigned long long *p) {
-  if (threadIdx.x == 0) *p = 0ull;
+  if (!qctr) return;
+  if (blockIdx.x == 0) queue_reset(qctr, (int)threadIdx.x, grid);
+  unsigned long long *evals = qctr + FORCE_TOTALS + 2;
+  for (int64_t j = k; j < 2 * grid; j += (int64_t)gridDim.x * blockDim.x) evals[j] = 0;
 }
 
 __global__ void k_kick(int64_t nleaves, const hsr_node *cn,
@@ -725,11 +793,46 @@ std::string force_shapes_built() {
   return out;
 }
 
+// List entries per work item when the caller sets none: CHUNK_MAX, halved
+// while the lists would give the chip fewer than ITEMS_PER_CU items per
+// compute unit, down to one tile.  A wave works through its item alone, so a
+// load whose leaves are few or short leaves most of the chip idle, and the
+// rest waiting for the longest list, unless the lists are cut finer; above
+// the line the items outnumber the resident waves (20 per compute unit)
+// several times and a finer cut only adds target loads and partial sums
+// (8192 measured 0.5% faster for the leaf kernel and 2% for the adjoint than
+// 16384 at 256^3).  Leaf kernel and fused adjoint with 8192 and with this
+// rule (queue.h's queue both times): 0.62 and 0.18, 1.31 and 0.46 ms on a
+// 50^3 Plummer mix with leaves of 128; 0.87 and 0.47 ms (leaf kernel) at 64^3.
+// The partial sums the cut makes (12 bytes per target and item of a leaf
+// with several) stay below PART_MAX bytes.
+constexpr int64_t CHUNK_MAX = 8192, CHUNK_MIN = 256, ITEMS_PER_CU = 160;
+constexpr int64_t PART_MAX = (int64_t)1 << 28;
+
+static int64_t auto_chunk(const hsr_ctx *c) {
+  const int64_t want = (int64_t)std::max(1, c->num_cus) * ITEMS_PER_CU;
+  int64_t chunk = CHUNK_MAX;
+  while (chunk > CHUNK_MIN && c->lists.nentries / chunk < want &&
+         c->lists.pairs / (chunk / 2) <= PART_MAX / 12)
+    chunk >>= 1;
+  return chunk;
+}
+
+static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk);
+
 hsr_status force_plan(hsr_ctx *c) {
+  if (c->tuning.chunk > 0) return force_plan_chunk(c, c->tuning.chunk);
+  const int64_t chunk = auto_chunk(c);
+  hsr_status s = force_plan_chunk(c, chunk);
+  // a cap on the plan's memory that the finer cut exceeds
+  if (s == HSR_ERR_NOMEM && chunk < CHUNK_MAX) s = force_plan_chunk(c, CHUNK_MAX);
+  return s;
+}
+
+static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   hipStream_t st = c->stream;
   ListState &LS = c->lists;
   const int64_t nl = LS.nleaves;
-  const int64_t chunk = c->tuning.chunk > 0 ? c->tuning.chunk : 8192;
   LS.chunk = chunk;
   if (nl == 0) {
     LS.nitems = 0;
@@ -768,15 +871,13 @@ hsr_status force_plan(hsr_ctx *c) {
   const int64_t nitems = tail[0] + tail[1];
   const int64_t nmulti = tail[2] + tail[3];
   const int64_t npart = tail[4] + tail[5];
-  // the item sort and the item ids are 32-bit
+  // the item ids are 32-bit
   if (nitems >= (int64_t)INT32_MAX) {
     hsr_set_error("force plan: " + std::to_string(nitems) +
                   " work items (2^31 or more); raise tuning.chunk");
     return HSR_ERR_NOMEM;
   }
-  const int64_t plan_bytes = (int64_t)sizeof(Item) * 2 * (nitems + 1) +
-                             (int64_t)(sizeof(uint64_t) + sizeof(int32_t)) * 2 * (nitems + 1) +
-                             (int64_t)sizeof(float) * npart;
+  const int64_t plan_bytes = (int64_t)sizeof(Item) * 2 * (nitems + 1) + (int64_t)sizeof(float) * npart;
   if (c->tuning.max_plan_bytes > 0 && plan_bytes > c->tuning.max_plan_bytes) {
     hsr_set_error("force plan: needs " + std::to_string(plan_bytes) + " bytes, above tuning.max_plan_bytes (" +
                   std::to_string(c->tuning.max_plan_bytes) + ")");
@@ -785,27 +886,20 @@ hsr_status force_plan(hsr_ctx *c) {
   LS.nitems = nitems;
   LS.nmulti = nmulti;
   HSR_HIP(dbuf_reserve(LS.items, sizeof(Item) * 2 * (nitems + 1)));
-  HSR_HIP(dbuf_reserve(LS.item_keys, (sizeof(uint64_t) + sizeof(int32_t)) * 2 * (nitems + 1) + 256));
+  HSR_HIP(dbuf_reserve(LS.item_keys, sizeof(uint32_t) * 2 * NCLASS));
   HSR_HIP(dbuf_reserve(LS.part, sizeof(float) * std::max<int64_t>(npart, 1)));
   Item *items_tmp = dptr<Item>(LS.items) + (nitems + 1);
   Item *items = dptr<Item>(LS.items);
-  uint64_t *keys = dptr<uint64_t>(LS.item_keys);
-  uint64_t *keys2 = keys + (nitems + 1);
-  int32_t *vals = reinterpret_cast<int32_t *>(keys2 + (nitems + 1));
-  int32_t *vals2 = vals + (nitems + 1);
+  uint32_t *hist = dptr<uint32_t>(LS.item_keys);
+  k_zero_classes<<<1, NCLASS, 0, st>>>(hist);
   k_item_fill<<<nblk(nl, 256), 256, 0, st>>>(nl, ent_ptr, chunk, nchunk, item_base, pbase, cn, leaves,
-                                             items_tmp, keys, vals, multi, mpos, mflag);
+                                             items_tmp, hist, multi, mpos, mflag);
   // heaviest items first
-  size_t tmp = 0;
-  HSR_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, tmp, keys, keys2, vals, vals2, (int)nitems, 0, 64, st));
-  HSR_HIP(dbuf_reserve(c->s.cub, tmp + 256));
-  HSR_HIP(hipcub::DeviceRadixSort::SortPairsDescending(c->s.cub.p, tmp, keys, keys2, vals, vals2, (int)nitems, 0, 64, st));
-  k_item_permute<<<nblk(nitems, 256), 256, 0, st>>>(nitems, items_tmp, vals2, items);
+  k_item_order<<<nblk(nitems, 256), 256, 0, st>>>(nitems, items_tmp, hist, hist + NCLASS, items);
   // device-resident counts for the persistent launch
   int64_t hc[2] = {nitems, nmulti};
   HSR_HIP(hipMemcpyAsync(counts, hc, sizeof(hc), hipMemcpyHostToDevice, st));
   HSR_HIP(stream_wait(st));
-  HSR_HIP(dbuf_reserve(c->s.qctr, 64));
   LS.multi = multi;
   LS.counts = counts;
   LS.leaf_pbase = pbase;
@@ -823,6 +917,15 @@ hsr_status force_plan(hsr_ctx *c) {
 
 static hsr_status force_enqueue(hsr_ctx *c, float *fx, float *fy, float *fz,
                                 bool timed);
+
+static_assert(FORCE_TOTALS >= QWORDS, "pair totals lie behind the queue's counters");
+
+// The persistent grid does not depend on the item count (waves beyond the
+// items leave at once), so a captured launch fits any list.
+static int64_t force_grid(const hsr_ctx *c) {
+  const int wpc = c->tuning.waves_per_cu > 0 ? c->tuning.waves_per_cu : 32;
+  return (int64_t)std::max(1, c->num_cus) * wpc;
+}
 
 static unsigned reduce_grid(const hsr_ctx *c) {
   unsigned g = 256;
@@ -842,6 +945,7 @@ hsr_status force_run(hsr_ctx *c, float *fx, float *fy, float *fz) {
     hsr_set_error("HSR_LAW_SR_INTERP: no table (call hsr_set_law_table first)");
     return HSR_ERR_STATE;
   }
+  HSR_HIP(dbuf_reserve(c->s.qctr, sizeof(unsigned long long) * (FORCE_TOTALS + 2 + 2 * (size_t)force_grid(c))));
   if (!c->tuning.use_graph) return force_enqueue(c, fx, fy, fz, true);
   const ListState &LS = c->lists;
   const uintptr_t sig[20] = {(uintptr_t)fx, (uintptr_t)fy, (uintptr_t)fz, (uintptr_t)c->tree.n,
@@ -891,22 +995,19 @@ static hsr_status force_enqueue(hsr_ctx *c, float *fx, float *fy, float *fz,
   const int64_t n = c->tree.n;
   ListState &LS = c->lists;
   if (timed) c->kernel_timed = false;
-  if (n > 0)
-    k_fill3<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, fx, fy, fz);
-  if (LS.nleaves == 0 || LS.nitems == 0) return HSR_OK;
+  const bool work = LS.nleaves > 0 && LS.nitems > 0;
+  const int64_t grid = force_grid(c);
   unsigned long long *qctr = dptr<unsigned long long>(c->s.qctr);
-  k_zero_u64<<<1, 64, 0, st>>>(qctr);
-  k_zero_u64<<<1, 64, 0, st>>>(qctr + 1);
-  k_zero_u64<<<1, 64, 0, st>>>(qctr + 2);
+  if (n > 0 || work)
+    k_fill3<<<(unsigned)std::max<int64_t>(1, (n + 255) / 256), 256, 0, st>>>(n, fx, fy, fz,
+                                                                             work ? qctr : nullptr, grid);
+  if (!work) return HSR_OK;
+  unsigned long long *totals = qctr + FORCE_TOTALS, *evals = totals + 2;
   LawArgs A = law_args(c->law);
   A.cull = c->tuning.cull_off ? 0 : 1;
   int R, U, T;
   force_shape(c->tuning, &R, &U, &T);
   A.pmax = c->tuning.force_pass == 32 * R ? 32 * R : 64 * R;
-  const int wpc = c->tuning.waves_per_cu > 0 ? c->tuning.waves_per_cu : 32;
-  // the persistent grid does not depend on the item count (waves beyond the
-  // items leave at their first pop), so a captured launch fits any list
-  const int64_t grid = (int64_t)std::max(1, c->num_cus) * wpc;
   const hsr_node *cn = dptr<hsr_node>(c->tree.canon_nodes);
   const int32_t *leaves = dptr<int32_t>(LS.leaves);
   const Item *items = dptr<Item>(LS.items);
@@ -916,7 +1017,7 @@ static hsr_status force_enqueue(hsr_ctx *c, float *fx, float *fy, float *fz,
 #define LAUNCH(LK, ORD, GRD, RR, UU, TT)                                              \
   k_force<LK, ORD, GRD, RR, UU, TT><<<(unsigned)grid, 64, 0, st>>>(cn, leaves, items, LS.counts, \
       dptr<int32_t>(LS.jidx), dptr<PJ>(c->tree.pj), dptr<int32_t>(LS.iperm), A, qctr, fx, fy, fz, \
-      part, qctr + 1)
+      part, evals)
 #define SHAPES(ORD)                                                                      \
   if (R == 2 && U == 1 && T == 256) LAUNCH(LAWK_POLY, ORD, false, 2, 1, 256);            \
   else if (R == 2 && U == 4 && T == 256) LAUNCH(LAWK_POLY, ORD, false, 2, 4, 256);       \
@@ -949,9 +1050,9 @@ static hsr_status force_enqueue(hsr_ctx *c, float *fx, float *fy, float *fz,
   // a grid over the device-resident multi-chunk count (which may be 0): a
   // wave per multi-chunk leaf, the grid rounded up to a power of two so a
   // captured force phase serves later lists unless their count outgrows it
-  k_reduce_chunks<<<reduce_grid(c), 64, 0, st>>>(
+  k_reduce_chunks<<<reduce_grid(c) + 1, 64, 0, st>>>(
       cn, leaves, LS.multi, LS.counts + 1, LS.leaf_pbase, LS.leaf_nchunk, dptr<int32_t>(LS.iperm), part,
-      fx, fy, fz);
+      fx, fy, fz, LS.counts, grid, evals, totals);
   HSR_HIP(hipGetLastError());
   return HSR_OK;
 }

@@ -133,7 +133,7 @@ struct ListState {
   DBuf ent_ptr;               // int64 [nleaves+1] list-entry CSR
   DBuf jidx;                  // int32 [nentries] index into PJ
   DBuf items;                 // work items for the force kernel (sorted)
-  DBuf item_keys;             // sort scratch
+  DBuf item_keys;             // work classes: item counts and slots given out
   DBuf plan;                  // per-leaf chunk plan
   DBuf part;                  // chunk partial forces of long lists
   int64_t nitems = 0, nmulti = 0, chunk = 0;
@@ -221,8 +221,9 @@ struct hsr_ctx {
   bool kernel_timed = false;
   // force phase captured as a hipGraph (tuning.use_graph)
   int64_t lists_gen = 0;
-  int64_t evaluated_pairs = 0;  // last force phase, culled entries excluded
-  int64_t unmasked_pairs = 0;   // of which unit-mass entries inside the cutoff
+  // pairs the last force phase evaluated (culled entries excluded), and of
+  // which unit-mass entries inside the cutoff
+  int64_t pair_counts[2] = {0, 0};
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   int64_t graph_gen = -1;       // -1: the captured force phase is stale
@@ -250,6 +251,9 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
 hsr_status lists_build_device(hsr_ctx *c, const float *min_force,
                               const float *max_force);
 hsr_status force_plan(hsr_ctx *c);
+// where the force phase's pair totals (evaluated, unmasked) lie in its work
+// queue's buffer (s.qctr, in 8-byte words)
+constexpr int FORCE_TOTALS = 1024;
 // the leaf kernel's shape (targets per lane, entries per unrolled step,
 // entries per LDS tile) for a tuning, 0 fields taking the defaults; whether
 // that shape is built for a law; the built shapes as text
