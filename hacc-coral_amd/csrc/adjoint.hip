@@ -27,6 +27,7 @@
 //                 hold the leaf); pseudo pass per (target leaf, pseudo
 //                 segment).  Used when W does not fit in device memory.
 #include "hsr_internal.h"
+#include "passes.h"
 #include "queue.h"
 #include "wave.h"
 
@@ -58,6 +59,7 @@ struct AdjLaw {
   int order;
   int cull;     // drop entries farther than the cutoff from a pass's target box
   float cull2;  // squared box distance beyond which every pair is masked
+  int thin;     // few waves share a SIMD: fewer, wider passes (pass_slots)
 };
 
 // Squared distance from p to the box [lo, hi] (0 inside).
@@ -88,6 +90,7 @@ AdjLaw adj_law(const ForceLawDev &D) {
   A.order = D.order;
   A.cull = 1;
   A.cull2 = (float)((double)D.rc2 * (1.0 + 1e-4));
+  A.thin = 0;
   return A;
 }
 
@@ -360,16 +363,6 @@ __device__ __forceinline__ float group_sum_last(float v) {
   return v;
 }
 
-// Targets of the next pass over a leaf: 128 while that many remain, then the
-// largest of 64, 32, 16, 8 that fits, then the rest (< 8).  With two targets
-// per lane each chunk fills groups of a power-of-two width exactly.
-__device__ __forceinline__ int64_t pass_size(int64_t rem) {
-  if (rem >= 64 * FR) return 64 * FR;
-  for (int64_t c = 32 * FR; c >= 4 * FR; c >>= 1)
-    if (rem >= c) return c;
-  return rem;
-}
-
 // A group's slice of the staged tile: every pair of its FR targets per lane
 // with each entry, the target sums B in registers, and the entry's source sum
 // W (over the group's lpg = LP lanes) written back into its tile slot.
@@ -469,12 +462,13 @@ adj_fused_body(const hsr_node *__restrict__ cn, const AItem *__restrict__ items,
     }
     const float4 padJ = make_float4(nd.xc[0] + 1000.f, nd.xc[1], nd.xc[2], 0.f);
     const float padI = nd.xc[0] + 3000.f;
-    // passes over the targets in power-of-two chunks (128, 64, ..., 8, rest)
-    // so that every pass fills its groups of lp = chunk / FR lanes
+    // passes over the targets, each of a power of two of slots in groups of
+    // lp = slots / FR lanes
     for (int64_t ib = 0, ni = 0; ib < cnt; ib += ni) {
       const bool first = ib == 0;
-      ni = pass_size(cnt - ib);
-      const int lp = max((int)(ni + FR - 1) / FR, 4);
+      const int slots = pass_slots<FR>(cnt - ib, 64 * FR, L.thin);
+      ni = min<int64_t>(slots, cnt - ib);
+      const int lp = slots / FR;
       const int G = 64 / lp;
       const int g = l / lp, tq = l & (lp - 1);
       float xi[FR], yi[FR], zi[FR], la[FR], lb[FR], lc[FR], am[FR], bx[FR], by[FR], bz[FR];
@@ -1186,6 +1180,7 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
   const PJ *pj = dptr<PJ>(c->tree.pj);
   AdjLaw L = adj_law(c->law);
   L.cull = c->tuning.cull_off ? 0 : 1;
+  L.thin = c->lists.thin;
   unsigned long long *q = dptr<unsigned long long>(A.qctr);
   float *part = dptr<float>(A.part);
   const int32_t *iperm = dptr<int32_t>(c->lists.iperm);

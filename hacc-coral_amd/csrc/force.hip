@@ -18,6 +18,7 @@
 // reads fall in distinct banks).  Chunk partials of long lists are summed in
 // chunk order afterwards, so results are bitwise reproducible.
 #include "hsr_internal.h"
+#include "passes.h"
 #include "queue.h"
 #include "wave.h"
 
@@ -34,8 +35,8 @@ namespace {
 // i_per_lane, unroll, tile).
 constexpr int DEF_R = 2, DEF_U = 2, DEF_T = 256;
 constexpr int GMAX = 16;      // at most 16 lane groups (>= 4 lanes each)
-// Passes hold a power of two of at least 4 R targets, or fewer than 4 R, so
-// the group count G = 64 / max(ceil(targets / R), 4) is 1, 2, 4, 8 or 16;
+// Passes hold a power of two of at least 4 R target slots, so the group
+// count G = 64 / (slots / R) is 1, 2, 4, 8 or 16;
 // the staged slices of a full tile must fit for each of them.  A group's
 // slice holds its unmasked entries (a multiple of UU) and its masked ones
 // rounded up to UU: at most ceil(entries / G) + UU - 1 slots.
@@ -71,6 +72,7 @@ struct LawArgs {
   int cull;        // drop entries farther than the cutoff from the leaf's box
   float cull2;     // squared box distance beyond which every pair is masked
   int pmax;        // targets per pass (64 R or 32 R)
+  int thin;        // few waves share a SIMD: fewer, wider passes (pass_slots)
   float in2;       // squared farthest box distance below which every pair of
                    // the pass is inside the cutoff (the unmasked class)
   int unmasked;    // 1: unit-mass entries inside the cutoff skip mask and mass
@@ -140,16 +142,6 @@ __device__ __forceinline__ float poly_tail(const LawArgs &L, float s) {
   q = fmaf(q, s, L.c[2]);
   q = fmaf(q, s, L.c[1]);
   return q;
-}
-
-// Targets of the next pass over a leaf: 64 R while that many remain, then
-// the largest power of two of at least 4 R that fits, then the rest.
-template <int R>
-__device__ __forceinline__ int64_t pass_size(int64_t rem, int pmax) {
-  if (rem >= pmax) return pmax;
-  for (int64_t c = pmax >> 1; c >= 4 * R; c >>= 1)
-    if (rem >= c) return c;
-  return rem;
 }
 
 // Waves per SIMD the register allocation of the leaf kernel targets (0: the
@@ -243,22 +235,22 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
     // padding entries: far enough to be masked, near enough to keep every
     // intermediate finite
     const float4 pad = make_float4(nd.xc[0] + 1000.f, nd.xc[1], nd.xc[2], 0.f);
-    // passes over the targets in power-of-two chunks (128, 64, ..., 8, rest)
-    // so that every pass fills its groups of lpg = chunk / R lanes
+    // passes over the targets, each of a power of two of slots in groups of
+    // lpg = slots / R lanes
     for (int64_t ib = 0, nib = 0; ib < cnt; ib += nib) {
-      nib = pass_size<R>(cnt - ib, L.pmax);
+      const int slots = pass_slots<R>(cnt - ib, L.pmax, L.thin);
+      nib = min<int64_t>(slots, cnt - ib);
       const int ni = (int)nib;
-      const int lpg = max((ni + R - 1) / R, 64 / GMAX);
-      const int G = max(1, 64 / lpg);
-      const int g = l / lpg, tq = l - g * lpg;
-      const bool active = g < G;
+      const int lpg = slots / R;
+      const int G = 64 / lpg;
+      const int g = l / lpg, tq = l & (lpg - 1);
       float xi[R], yi[R], zi[R], ax[R], ay[R], az[R];
       // the pass's targets (in the leaf's target order) and their box
       float bmin[3] = {INFINITY, INFINITY, INFINITY}, bmax[3] = {-INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int ii = tq + r * lpg;
-        const bool v = active && ii < ni;
+        const bool v = ii < ni;
         const PJ p = pj[iperm[off + ib + (v ? ii : 0)]];
         xi[r] = v ? p.x : 1e30f;
         yi[r] = v ? p.y : 1e30f;
@@ -354,7 +346,7 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
         ev += (int64_t)nK * ni;
         evu += (int64_t)splitA * ni;
         __syncthreads();
-        if (active) {
+        {
           const float4 *tp = tile + g * stride;
           for (int k = 0; k < tA; k += UNROLL) {
 #pragma unroll
@@ -381,7 +373,7 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
       for (int q = l; q < 64 * R; q += 64) red[0][q] = red[1][q] = red[2][q] = 0.f;
       __syncthreads();
       for (int gg = 0; gg < G; ++gg) {
-        if (active && g == gg) {
+        if (g == gg) {
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             const int ii = tq + r * lpg;
@@ -685,6 +677,7 @@ LawArgs law_args(const ForceLawDev &D) {
   A.cull = 1;
   A.cull2 = (float)((double)D.rc2 * (1.0 + 1e-4));
   A.pmax = 64 * DEF_R;
+  A.thin = 0;
   // the same relative margin the other way: every pair of an entry whose
   // farthest box point is inside in2 passes the kernel's cutoff test
   A.in2 = (float)((double)D.rc2 * (1.0 - 1e-4));
@@ -701,7 +694,6 @@ LawArgs law_args(const ForceLawDev &D) {
 
 }  // namespace
 
-// Work items of the current lists (rebuilt after every hsr_lists call).
 // Target order inside each listed leaf: positions sorted along the leaf's
 // longest box edge (ties x > y > z; equal coordinates by position), so that
 // a pass's 128 targets span a slab of the leaf and the entries its box is
@@ -834,6 +826,9 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   ListState &LS = c->lists;
   const int64_t nl = LS.nleaves;
   LS.chunk = chunk;
+  // the lists were short of items for the chip: what waves there are run
+  // with few others on their SIMD
+  LS.thin = LS.nentries / CHUNK_MAX < (int64_t)std::max(1, c->num_cus) * 16;
   if (nl == 0) {
     LS.nitems = 0;
     return HSR_OK;
@@ -953,7 +948,7 @@ hsr_status force_run(hsr_ctx *c, float *fx, float *fy, float *fz) {
                              (uintptr_t)LS.leaves.p, (uintptr_t)LS.items.p, (uintptr_t)LS.counts,
                              (uintptr_t)LS.jidx.p, (uintptr_t)c->tree.pj.p, (uintptr_t)LS.iperm.p,
                              (uintptr_t)LS.part.p, (uintptr_t)LS.multi, (uintptr_t)LS.leaf_pbase,
-                             (uintptr_t)LS.leaf_nchunk, (uintptr_t)c->s.qctr.p, (uintptr_t)reduce_grid(c), 0, 0};
+                             (uintptr_t)LS.leaf_nchunk, (uintptr_t)c->s.qctr.p, (uintptr_t)reduce_grid(c), (uintptr_t)LS.thin, 0};
   bool same = c->graph_exec != nullptr && c->graph_gen != -1;
   for (int k = 0; k < 20 && same; ++k) same = c->graph_sig[k] == sig[k];
   const bool stale = !same;
@@ -1008,6 +1003,7 @@ static hsr_status force_enqueue(hsr_ctx *c, float *fx, float *fy, float *fz,
   int R, U, T;
   force_shape(c->tuning, &R, &U, &T);
   A.pmax = c->tuning.force_pass == 32 * R ? 32 * R : 64 * R;
+  A.thin = LS.thin;
   const hsr_node *cn = dptr<hsr_node>(c->tree.canon_nodes);
   const int32_t *leaves = dptr<int32_t>(LS.leaves);
   const Item *items = dptr<Item>(LS.items);

@@ -137,6 +137,7 @@ struct ListState {
   DBuf plan;                  // per-leaf chunk plan
   DBuf part;                  // chunk partial forces of long lists
   int64_t nitems = 0, nmulti = 0, chunk = 0;
+  bool thin = false;          // the lists do not fill the chip (pass_slots)
   int64_t plan_stride = 0;    // per-leaf plan arrays' stride (grows only)
   int64_t *multi = nullptr, *counts = nullptr, *leaf_pbase = nullptr;
   int32_t *leaf_nchunk = nullptr;
