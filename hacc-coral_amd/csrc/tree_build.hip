@@ -28,6 +28,8 @@ constexpr int CM_PER = CM_BLK / 64; // consecutive addends each lane composes
 constexpr int64_t CM_SMALL = 2048;  // nodes up to this size: one wave each
 constexpr int PB = 1024;            // partition block (256 threads x 4)
 constexpr int MAXHOP = 256;         // swap-chain hops before pointer jumping (default)
+constexpr int SUB_MAX = 2048;       // k_subtree's particles (= CM_SMALL)
+constexpr int NODE_SUB = 3;         // BNode.kind of its roots until it has run
 
 struct Counters {
   int64_t cm_blocks;      // big-node cm blocks allocated this level
@@ -41,6 +43,7 @@ struct Counters {
   int64_t next_small;     // and with count <= CM_SMALL
   int64_t next_leaf;      // and with count <= nd (leaves of the next level)
   int64_t ndegen;         // degenerate splits of this level
+  int64_t nsub;           // nodes of this level left to k_subtree
 };
 
 // ------------------------------------------------------------ helpers
@@ -936,7 +939,9 @@ __global__ void k_pj_particles(int64_t n, const float *xs, const float *ys, cons
 // ------------------------------------------------------------ partition
 __global__ void __launch_bounds__(64)
 k_part_plan(BNode *nodes, int64_t lb, int64_t le, bool unit, const sd_t *cms, int64_t nd,
-            float ppc, bool unit_ppm, int32_t *pnode, Counters *ctr) {
+            float ppc, bool unit_ppm, int32_t *pnode, Counters *ctr, int sub) {
+  // (sub >= 0: nodes of at most SUB_MAX particles are marked for k_subtree,
+  // with the copy their particles are in, and left alone)
   // one lane per node: its centre of mass and class (cm_finish_node,
   // classify_node), then a wave scan of the block counts of the splitting
   // nodes and one atomic per wave reserve their partition blocks; then the
@@ -945,11 +950,20 @@ k_part_plan(BNode *nodes, int64_t lb, int64_t le, bool unit, const sd_t *cms, in
   const int64_t t0 = lb + (int64_t)blockIdx.x * 64;
   const int64_t t = t0 + l;
   int64_t nb = 0;
+  bool mine = false;
   if (t < le) {
     BNode &n = nodes[t];
-    cm_finish_node(n, unit, cms + 4 * (t - lb));
-    if (classify_node(n, nd, ppc, unit_ppm)) nb = (n.count + PB - 1) / PB;
+    if (sub >= 0 && n.count > 0 && n.count <= SUB_MAX) {
+      n.kind = NODE_SUB;
+      n.blk0 = sub;
+      mine = true;
+    } else {
+      cm_finish_node(n, unit, cms + 4 * (t - lb));
+      if (classify_node(n, nd, ppc, unit_ppm)) nb = (n.count + PB - 1) / PB;
+    }
   }
+  const uint64_t subs = __ballot(mine);
+  if (l == 0 && subs) atomicAdd((unsigned long long *)&ctr->nsub, (unsigned long long)__popcll(subs));
   int64_t inc = nb;
   for (int o = 1; o < 64; o <<= 1) {
     const int64_t y = (int64_t)__shfl_up((long long)inc, o);
@@ -1305,10 +1319,8 @@ __global__ void k_make_children(BNode *nodes, int64_t lb, int64_t le, int64_t nd
 // ------------------------------------------------------------ finishing
 // Bottom-up: parent pseudo-particles from the children, left then right
 // (RCBForceTree.cxx:856-889 with TDPTS = 1), allocating-node and leaf counts.
-__global__ void k_bottom_up(BNode *nodes, int64_t lb, int64_t le, float ppc,
-                            const int32_t *Pfin, const float *Min) {
-  int64_t t = lb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= le) return;
+__device__ __forceinline__ void bottom_up_node(BNode *nodes, int64_t t, float ppc,
+                                               const int32_t *Pfin, const float *Min) {
   BNode &n = nodes[t];
   if (n.kind == NODE_LEAF) {
     n.sa = 0;
@@ -1337,6 +1349,12 @@ __global__ void k_bottom_up(BNode *nodes, int64_t lb, int64_t le, float ppc,
   n.ppm = ppm;
   n.sa = 1 + L.sa + R.sa;
   n.nleaf = L.nleaf + R.nleaf;
+}
+
+__global__ void k_bottom_up(BNode *nodes, int64_t lb, int64_t le, float ppc,
+                            const int32_t *Pfin, const float *Min) {
+  int64_t t = lb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t < le) bottom_up_node(nodes, t, ppc, Pfin, Min);
 }
 
 // Top-down: canonical ids (children get 1 + 2A and 2 + 2A, A = allocating
@@ -1405,6 +1423,503 @@ __global__ void k_box_of(const BNode *nodes, int64_t nb, int32_t *box_of,
   box_of[t] = root_box[u];
 }
 
+// ------------------------------------------------------------ subtrees
+// A node of at most SUB_MAX particles with unit masses is built to its leaves
+// by one workgroup, its particles in LDS: the level passes above it cost a
+// dozen launches and a host round trip a level, some 0.1 ms whatever they
+// hold, and the last levels of a tree -- nearly all of a small one -- hold
+// only such nodes.  The steps are the level passes', with the same arithmetic:
+// bbox and exact sums (a wave per node), centre of mass and class, ranks,
+// swap chains, children, then the bottom-up pass.  The working copy is only
+// read, so a launch that runs out of node slots is repeated with more.
+//
+// A workgroup takes 12 to 15 us a level (dependent integer chains and
+// barriers; 97 KB of LDS, one workgroup a compute unit), so it pays where
+// the levels it replaces are bound by their launches: builds of up to SUB_N
+// particles.  Build time without and with it: 0.99 and 0.63 ms for 12k
+// particles (leaves of 32), 1.93 and 1.62 ms for 365k (leaves of 128), but
+// 3.95 and 4.10 ms for 2.5M (leaves of 256), 9.78 and 10.58 ms for 18M.
+constexpr int SUB_T = 1024;
+constexpr int64_t SUB_N = (int64_t)1 << 20;
+constexpr int SUB_LEVELS = 48;  // levels of a subtree (a deeper one sends the build
+                                // to the level passes)
+
+struct SubCtr {
+  int64_t next;      // next free node slot
+  int32_t overflow;  // a workgroup found no slots
+  int32_t deep;      // a subtree has more than SUB_LEVELS levels
+  int64_t depth;     // deepest level used
+};
+
+struct SubArrays {
+  const float *x[3], *y[3], *z[3];  // the two working copies, the caller's arrays
+  const int32_t *p[2];
+};
+
+// The marked nodes (ids below nb) in a list, with their copy's number.
+__global__ void k_sub_gather(const BNode *nodes, int64_t nb, int2 *list, int32_t *count) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const bool mine = t < nb && nodes[t].kind == NODE_SUB;
+  const uint64_t bal = __ballot(mine);
+  int32_t base = 0;
+  if (lane_id() == 0 && bal) base = atomicAdd(count, (int32_t)__popcll(bal));
+  base = readlane_i32(base, 0);
+  if (mine) list[base + __popcll(bal & lanemask_lt())] = make_int2((int)t, (int)nodes[t].blk0);
+}
+
+__global__ void k_sub_init(SubCtr *c, int64_t next, int32_t *count) {
+  if (threadIdx.x == 0) {
+    c->next = next;
+    c->overflow = c->deep = 0;
+    c->depth = 0;
+    if (count) *count = 0;
+  }
+}
+
+__global__ void __launch_bounds__(SUB_T)
+k_subtree(BNode *nodes, const int2 *__restrict__ list, SubArrays A, int64_t nd, float ppc,
+          int64_t cap, SubCtr *ctr, int32_t *__restrict__ Pfin, float *__restrict__ xs,
+          float *__restrict__ ys, float *__restrict__ zs, float *__restrict__ ms) {
+  constexpr int PER = SUB_MAX / SUB_T;   // elements a thread moves
+  constexpr int NW = SUB_T / 64;
+  constexpr int WORDS = SUB_MAX / 64;
+  constexpr uint16_t DONE = 0xffff;      // element's node has stopped splitting
+  enum { D_LEAF = 3, D_DEGEN = 4 };
+  __shared__ float C[3][SUB_MAX];
+  __shared__ int32_t perm[SUB_MAX];
+  __shared__ uint16_t node_of[SUB_MAX], nis[SUB_MAX];
+  // the forward pass's ranks and level tables; the bottom-up pass's sums
+  __shared__ uint16_t pool[6 * SUB_MAX];
+#define SUB_IDX(i) pool[i]
+#define SUB_RIGHTS(i) pool[SUB_MAX + (i)]
+#define SUB_OFF(c, k) pool[(2 + (c)) * SUB_MAX + (k)]
+#define SUB_CNT(c, k) pool[(4 + (c)) * SUB_MAX + (k)]
+  // every node of the subtree in level order: members, and the first child
+  __shared__ uint16_t acnt[2 * SUB_MAX], achild[2 * SUB_MAX];
+  constexpr uint16_t CH_LEAF = 0xffff, CH_DEGEN = 0xfffe;
+  // partial sums of the top levels' nodes, SUB_CH elements each
+  constexpr int SUB_CH = 128, NTOP = 8, NPART = SUB_MAX / SUB_CH + NTOP;
+  __shared__ uint64_t pu[NPART][3];
+  __shared__ int32_t pt[NPART][3], pbad[NPART];
+  __shared__ float pmn[NPART][3], pmx[NPART][3];
+  __shared__ uint8_t ndim[SUB_MAX];
+  __shared__ float npiv[SUB_MAX];
+  __shared__ uint64_t mask[WORDS], smask[WORDS];   // key < pivot; node splits
+  __shared__ int32_t wpre[WORDS + 1], spre[WORDS + 1];
+  __shared__ int64_t lbase[SUB_LEVELS];
+  __shared__ int32_t lcnt[SUB_LEVELS], lfirst[SUB_LEVELS];
+  __shared__ int64_t base_sh;
+  __shared__ int32_t stop_sh;
+  const int t = threadIdx.x, w = t >> 6, l = lane_id();
+  const int2 item = list[blockIdx.x];
+  const int64_t root = item.x;
+  const int n = (int)nodes[root].count;
+  const int64_t goff = nodes[root].offset;
+  const int depth0 = nodes[root].depth;
+  {
+    const float *x = A.x[item.y], *y = A.y[item.y], *z = A.z[item.y];
+    for (int e = t; e < n; e += SUB_T) {
+      C[0][e] = x[goff + e];
+      C[1][e] = y[goff + e];
+      C[2][e] = z[goff + e];
+      perm[e] = item.y == 2 ? (int32_t)(goff + e) : A.p[item.y][goff + e];
+      node_of[e] = 0;
+    }
+  }
+  if (t == 0) {
+    SUB_OFF(0, 0) = 0;
+    SUB_CNT(0, 0) = (uint16_t)n;
+  }
+  __syncthreads();
+  // elements < p with key < pivot (p up to SUB_MAX)
+  auto lefts = [&](int p) {
+    return wpre[p >> 6] + ((p & 63) ? __popcll(mask[p >> 6] & (~0ull >> (64 - (p & 63)))) : 0);
+  };
+  int64_t base = root;
+  int nn = 1, cur = 0, lev = 0, first = 0;
+  while (nn > 0) {
+    if (lev == SUB_LEVELS) {
+      if (t == 0) ctr->deep = 1;
+      return;
+    }
+    if (t == 0) {
+      lbase[lev] = base;
+      lcnt[lev] = nn;
+      lfirst[lev] = first;
+    }
+    // ---- bbox, exact sums, centre of mass, class: a wave per node, at the
+    // top levels after a wave per SUB_CH elements of it
+    const bool top = nn <= NTOP;
+    if (top) {
+      int p = 0;
+      for (int k = 0; k < nn; ++k) {
+        const int off = SUB_OFF(cur, k), c = SUB_CNT(cur, k);
+        for (int i0 = 0; i0 < c; i0 += SUB_CH, ++p) {
+          if (p % NW != w) continue;
+          float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+          LaneSum ls[3];
+          for (int i = i0 + l; i < min(c, i0 + SUB_CH); i += 64) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              const float v = C[d][off + i];
+              mn[d] = fminf(mn[d], v);
+              mx[d] = fmaxf(mx[d], v);
+              lane_sum_add(ls[d], v);
+            }
+          }
+          int32_t bads = 0;
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            mn[d] = wave_min_f32(mn[d]);
+            mx[d] = wave_max_f32(mx[d]);
+            int32_t tl;
+            bool bad;
+            const uint64_t tot = wave_lane_sum(ls[d], tl, bad);
+            if (bad) bads |= 1 << d;
+            if (l == 0) {
+              pu[p][d] = tot;
+              pt[p][d] = tl;
+              pmn[p][d] = mn[d];
+              pmx[p][d] = mx[d];
+            }
+          }
+          if (l == 0) pbad[p] = bads;
+        }
+      }
+      __syncthreads();
+    }
+    for (int k = w; k < nn; k += NW) {
+      const int off = SUB_OFF(cur, k), c = SUB_CNT(cur, k);
+      float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+      LaneSum ls[3];
+      if (top) {
+        int p = 0;
+        for (int j = 0; j < k; ++j) p += (SUB_CNT(cur, j) + SUB_CH - 1) / SUB_CH;
+        if (l < (c + SUB_CH - 1) / SUB_CH) {
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            mn[d] = pmn[p + l][d];
+            mx[d] = pmx[p + l][d];
+            ls[d].u = pu[p + l][d];
+            ls[d].t = pt[p + l][d];
+            ls[d].bad = (pbad[p + l] >> d) & 1;
+            if (ls[d].bad) ls[d].u = 0;
+          }
+        }
+      } else {
+        for (int i = l; i < c; i += 64) {
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            const float v = C[d][off + i];
+            mn[d] = fminf(mn[d], v);
+            mx[d] = fmaxf(mx[d], v);
+            lane_sum_add(ls[d], v);
+          }
+        }
+      }
+      sd_t S = sd_zero();  // lane d < 3: the sum of dimension d
+      int rounds = 0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        mn[d] = wave_min_f32(mn[d]);
+        mx[d] = wave_max_f32(mx[d]);
+        int32_t tl;
+        bool bad;
+        const uint64_t tot = wave_lane_sum(ls[d], tl, bad);
+        if (bad) rounds |= 1 << d;
+        else if (l == d) S = sd_from_units(tot, tl);
+      }
+#pragma unroll 1
+      for (int d = 0; d < 3; ++d) {  // the sums that round, in order
+        if (!((rounds >> d) & 1)) continue;
+        sd_t Sd = sd_zero();
+        sd_block(Sd, &C[d][off], c);
+        if (l == d) S = Sd;
+      }
+      const float q = l < 3 ? sd_div_to_f32(S, sd_from_units((uint64_t)c, 0)) : 0.f;
+      const float xc[3] = {__shfl(q, 0), __shfl(q, 1), __shfl(q, 2)};
+      if (l == 0) {
+        BNode N;  // in registers: a load would wait for the node's own stores
+        N.count = c;
+        for (int d = 0; d < 3; ++d) {
+          N.xmin[d] = mn[d];
+          N.xmax[d] = mx[d];
+          N.xc[d] = xc[d];
+        }
+        N.split_d = 0;
+        N.tdr = 0.f;
+        const bool split = classify_node(N, nd, ppc, true);
+        BNode &G = nodes[base + k];
+        for (int d = 0; d < 3; ++d) {
+          G.xmin[d] = mn[d];
+          G.xmax[d] = mx[d];
+          G.xc[d] = xc[d];
+        }
+        G.kind = N.kind;
+        G.split_d = N.split_d;
+        G.cl = G.cr = -1;
+        // the bottom-up pass's tdr of split nodes is the same expression
+        G.tdr = ppc * pptdr_dev(mn, mx, xc);
+        if (!split) G.ppm = N.ppm;
+        acnt[first + k] = (uint16_t)c;
+        achild[first + k] = CH_LEAF;
+        ndim[k] = split ? (uint8_t)N.split_d : (uint8_t)D_LEAF;
+        if (split) npiv[k] = N.split_d == 0 ? xc[0] : (N.split_d == 1 ? xc[1] : xc[2]);
+      }
+    }
+    __syncthreads();
+    // ---- leaves leave; the others' elements against their node's pivot
+    bool left[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = u * SUB_T + t;
+      const int k = e < n ? node_of[e] : DONE;
+      left[u] = false;
+      if (k != DONE) {
+        if (ndim[k] == D_LEAF) {
+          Pfin[goff + e] = perm[e];
+          xs[goff + e] = C[0][e];
+          ys[goff + e] = C[1][e];
+          zs[goff + e] = C[2][e];
+          ms[goff + e] = 1.f;
+          node_of[e] = DONE;
+        } else {
+          left[u] = C[ndim[k]][e] < npiv[k];
+        }
+      }
+      const uint64_t bal = __ballot(left[u]);
+      if (l == 0) mask[u * NW + w] = bal;
+    }
+    __syncthreads();
+    if (w == 0) {  // exclusive prefix of the words' counts
+      const int c = l < WORDS ? __popcll(mask[l]) : 0;
+      int inc = c;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o);
+        if (l >= o) inc += y;
+      }
+      if (l < WORDS) wpre[l] = inc - c;
+      if (l == WORDS - 1) wpre[WORDS] = inc;
+    }
+    __syncthreads();
+    // ---- left counts; which nodes split
+    for (int k0 = 0; k0 < SUB_MAX; k0 += SUB_T) {
+      const int k = k0 + t;
+      bool split = false;
+      if (k < nn && ndim[k] != D_LEAF) {
+        const int off = SUB_OFF(cur, k), c = SUB_CNT(cur, k);
+        const int is = lefts(off + c) - lefts(off);
+        nis[k] = (uint16_t)is;
+        BNode &N = nodes[base + k];
+        N.is = is;
+        split = is > 0 && is < c;
+        if (!split) {
+          N.kind = NODE_DEGEN;
+          ndim[k] = D_DEGEN;
+          achild[first + k] = CH_DEGEN;
+        }
+      }
+      const uint64_t bal = __ballot(split);
+      if (l == 0) smask[(k0 >> 6) + w] = bal;
+    }
+    __syncthreads();
+    if (w == 0) {
+      const int c = l < WORDS ? __popcll(smask[l]) : 0;
+      int inc = c;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o);
+        if (l >= o) inc += y;
+      }
+      if (l < WORDS) spre[l] = inc - c;
+      if (l == WORDS - 1) {
+        spre[WORDS] = inc;
+        int64_t b = 0;
+        int stop = 0;
+        if (inc > 0) {
+          b = (int64_t)atomicAdd((unsigned long long *)&ctr->next, 2ull * (unsigned)inc);
+          if (b + 2 * inc > cap) {
+            ctr->overflow = 1;
+            stop = 1;
+          }
+        }
+        base_sh = b;
+        stop_sh = stop;
+      }
+    }
+    __syncthreads();
+    if (stop_sh) return;
+    const int nsplit = spre[WORDS];
+    const int64_t nbase = base_sh;
+    // ---- ranks (k_part_rank)
+    int dst[PER];
+    int nk[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = u * SUB_T + t;
+      const int k = e < n ? node_of[e] : DONE;
+      nk[u] = k;
+      dst[u] = 0;
+      if (k == DONE) continue;
+      if (ndim[k] == D_DEGEN) {  // no element moves
+        Pfin[goff + e] = perm[e];
+        xs[goff + e] = C[0][e];
+        ys[goff + e] = C[1][e];
+        zs[goff + e] = C[2][e];
+        ms[goff + e] = 1.f;
+        node_of[e] = DONE;
+        nk[u] = DONE;
+        continue;
+      }
+      const int off = SUB_OFF(cur, k), p = e - off, r = lefts(e) - lefts(off);
+      if (left[u]) {
+        SUB_IDX(off + r) = (uint16_t)p;
+        dst[u] = r;
+      } else {
+        SUB_RIGHTS(off + p - r) = (uint16_t)p;
+        dst[u] = p >= nis[k] ? p : -1;
+      }
+    }
+    __syncthreads();
+    // ---- swap chains (k_part_chain), then every element's value in registers
+    float v[PER][3];
+    int32_t vp[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = u * SUB_T + t;
+      if (nk[u] == DONE) continue;
+      const int k = nk[u];
+      const int off = SUB_OFF(cur, k);
+      const uint32_t is = nis[k], cnt = SUB_CNT(cur, k), nr = cnt - is;
+      if (dst[u] < 0) {
+        uint32_t j = (uint32_t)(e - off);
+        for (;;) {
+          const uint32_t f = SUB_IDX(off + j);  // f > j
+          if (f >= is) {
+            dst[u] = (int)f;
+            break;
+          }
+          const uint32_t step = f - j;  // keys >= pivot below f
+          const uint32_t lim = step < nr ? SUB_RIGHTS(off + step) : cnt;
+          const uint32_t x = f + ((is - f + step - 1u) / step) * step;
+          if (x < lim) {
+            dst[u] = (int)x;
+            break;
+          }
+          j = f + ((lim - 1u - f) / step) * step;
+        }
+      }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) v[u][d] = C[d][e];
+      vp[u] = perm[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if (nk[u] == DONE) continue;
+      const int k = nk[u];
+      const int o = SUB_OFF(cur, k) + dst[u];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) C[d][o] = v[u][d];
+      perm[o] = vp[u];
+      const int r = spre[k >> 6] + ((k & 63) ? __popcll(smask[k >> 6] & (~0ull >> (64 - (k & 63)))) : 0);
+      node_of[o] = (uint16_t)(2 * r + (dst[u] >= (int)nis[k] ? 1 : 0));
+    }
+    // ---- children (k_make_children)
+    for (int k = t; k < nn; k += SUB_T) {
+      if (!((smask[k >> 6] >> (k & 63)) & 1ull)) continue;
+      const int r = spre[k >> 6] + ((k & 63) ? __popcll(smask[k >> 6] & (~0ull >> (64 - (k & 63)))) : 0);
+      const int off = SUB_OFF(cur, k), c = SUB_CNT(cur, k), is = nis[k];
+      achild[first + k] = (uint16_t)(first + nn + 2 * r);
+      SUB_OFF(cur ^ 1, 2 * r) = (uint16_t)off;
+      SUB_CNT(cur ^ 1, 2 * r) = (uint16_t)is;
+      SUB_OFF(cur ^ 1, 2 * r + 1) = (uint16_t)(off + is);
+      SUB_CNT(cur ^ 1, 2 * r + 1) = (uint16_t)(c - is);
+      BNode &N = nodes[base + k];
+      BNode &L = nodes[nbase + 2 * r];
+      BNode &R = nodes[nbase + 2 * r + 1];
+      N.cl = (int32_t)(nbase + 2 * r);
+      N.cr = (int32_t)(nbase + 2 * r + 1);
+      L.count = is;
+      L.offset = goff + off;
+      R.count = c - is;
+      R.offset = goff + off + is;
+      L.parent = R.parent = (int32_t)(base + k);
+      L.depth = R.depth = depth0 + lev + 1;
+      L.cl = L.cr = R.cl = R.cr = -1;
+      L.nblk = R.nblk = 0;
+    }
+    __syncthreads();
+    base = nbase;
+    first += nn;
+    nn = 2 * nsplit;
+    cur ^= 1;
+    ++lev;
+  }
+  // ---- bottom-up (k_bottom_up), deepest level first, in LDS: with unit
+  // masses a node's pseudo mass is its members outside degenerate nodes (sums
+  // of whole numbers below 2^24, exact in float)
+#define SUB_SA(i) pool[i]
+#define SUB_NLEAF(i) pool[2 * SUB_MAX + (i)]
+#define SUB_PM(i) pool[4 * SUB_MAX + (i)]
+  for (int v = lev - 1; v >= 0; --v) {
+    for (int k = t; k < lcnt[v]; k += SUB_T) {
+      const int i = lfirst[v] + k, ch = achild[i];
+      BNode &N = nodes[lbase[v] + k];
+      int a = 0, f = 1, m = acnt[i];
+      if (ch == CH_DEGEN) {
+        a = 1;
+        m = 0;
+      } else if (ch != CH_LEAF) {
+        a = 1 + SUB_SA(ch) + SUB_SA(ch + 1);
+        f = SUB_NLEAF(ch) + SUB_NLEAF(ch + 1);
+        m = SUB_PM(ch) + SUB_PM(ch + 1);
+      }
+      SUB_SA(i) = (uint16_t)a;
+      SUB_NLEAF(i) = (uint16_t)f;
+      SUB_PM(i) = (uint16_t)m;
+      N.sa = a;
+      N.nleaf = f;
+      if (ch != CH_LEAF) N.ppm = (float)m;
+    }
+    __syncthreads();
+  }
+  if (t == 0) atomicMax((unsigned long long *)&ctr->depth, (unsigned long long)(depth0 + lev - 1));
+#undef SUB_IDX
+#undef SUB_RIGHTS
+#undef SUB_OFF
+#undef SUB_CNT
+#undef SUB_SA
+#undef SUB_NLEAF
+#undef SUB_PM
+}
+
+// Canonical ids and leaf ranks of the nodes below the subtrees' roots (ids
+// from lb): k_top_down's steps summed up the path to the root's own values.
+__global__ void k_sub_top_down(BNode *nodes, int64_t lb, int64_t nb) {
+  const int64_t t = lb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t >= nb) return;
+  int64_t a = 0, rank = 0, first = 0;
+  bool right = false;
+  int64_t u = t;
+  while (u >= lb) {
+    const int64_t p = nodes[u].parent;
+    const BNode &P = nodes[p];
+    const bool r = P.cr == (int32_t)u;
+    const int64_t da = 1 + (r ? nodes[P.cl].sa : 0);
+    if (u == t) {
+      first = da;
+      right = r;
+    }
+    a += da;
+    if (!r) rank += nodes[P.cr].nleaf;
+    u = p;
+  }
+  a += nodes[u].a;
+  nodes[t].a = a;
+  nodes[t].leaf_rank = rank + nodes[u].leaf_rank;
+  nodes[t].canon = 1 + 2 * (a - first) + (right ? 1 : 0);
+}
+
 // ------------------------------------------------- quadrupole (TDPTS = 12)
 // Hardin and Sloane's 12-point spherical 4-design (the icosahedron's
 // vertices) as the reference tabulates it (RCBForceTree.cxx:229-272), in
@@ -1444,21 +1959,21 @@ __device__ __forceinline__ float pp12_term(float x, float y, float z, float w,
   return w * (odr0 + odr1 + odr2);
 }
 
-// pp<12> of every node of one BFS level (deepest level first), one thread
+// pp<12> of every node of one depth (deepest first), one thread
 // per (node, design point): leaves with count > 12 from their members
 // (RCBForceTree.cxx:787-797), split nodes from each child, left then right
 // -- its members when count <= 12, else its 12 pseudo-particles
 // (:856-889) -- accumulated in that order; degenerate nodes and leaves with
 // count <= 12 keep 0.  Reads the canonical nodes and the particles in tree
 // order; writes ppm12[12 * canonical id + j].
-__global__ void k_pp12_level(const BNode *nodes, int64_t lb, int64_t le,
+__global__ void k_pp12_level(const BNode *nodes, int64_t nb, int depth,
                              const int64_t *box_cbase, const int32_t *box_of,
                              hsr_node *cn, const float *xs, const float *ys,
                              const float *zs, const float *ms, float *ppm12) {
   const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t t = lb + g / 12;
+  const int64_t t = g / 12;
   const int j = (int)(g % 12);
-  if (t >= le) return;
+  if (t >= nb || nodes[t].depth != depth) return;
   const BNode &b = nodes[t];
   const int64_t k = box_cbase[box_of[t]] + b.canon;
   const hsr_node &o = cn[k];
@@ -1588,10 +2103,12 @@ inline unsigned nblk_for(int64_t n, int t) {
 
 }  // namespace
 
-hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
-                             const int64_t *box_off_h, const float *min_loc_h,
-                             const float *max_loc_h, const float *x,
-                             const float *y, const float *z, const float *m) {
+// The last levels by k_subtree where it can (subtrees), else by the level
+// passes alone.
+static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_off_h,
+                               const float *min_loc_h, const float *max_loc_h, const float *x,
+                               const float *y, const float *z, const float *m, bool subtrees,
+                               bool *too_deep) {
   hipStream_t st = c->stream;
   TreeState &T = c->tree;
   Scratch &S = c->s;
@@ -1614,7 +2131,7 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
   HSR_HIP(dbuf_reserve(S.b, sizeof(int32_t) * nn));  // dest
   HSR_HIP(dbuf_reserve(S.c, sizeof(int32_t) * nn));  // jmp
   HSR_HIP(dbuf_reserve(S.rights, sizeof(int32_t) * nn));
-  HSR_HIP(dbuf_reserve(S.counters, 2 * sizeof(Counters) + 64));
+  HSR_HIP(dbuf_reserve(S.counters, 2 * sizeof(Counters) + sizeof(SubCtr) + 64));
   HSR_HIP(dbuf_reserve(S.d, sizeof(int64_t) * (nboxes + 1) + sizeof(float) * 6 * nboxes + 64));
   // (the 64 spare bytes after the box table hold the unit-mass flag)
 
@@ -1629,6 +2146,7 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
   int32_t *jmp = dptr<int32_t>(S.c);
   int32_t *rights = dptr<int32_t>(S.rights);
   Counters *ctr2 = dptr<Counters>(S.counters);  // two sets, alternating by level
+  SubCtr *sub_ctr = reinterpret_cast<SubCtr *>(ctr2 + 2);
   // sorted arrays, written as nodes stop splitting
   for (DBuf *bb : {&T.xs, &T.ys, &T.zs, &T.ms})
     HSR_HIP(dbuf_reserve(*bb, sizeof(float) * nn));
@@ -1665,7 +2183,12 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
   int64_t active = n;
   Counters hc;
   int depth = 0;
-  bool run_big = true, run_small = true, run_leaf = true;
+  const bool use_sub = subtrees && unit && n <= SUB_N;
+  // whether the level holds nodes above CM_SMALL, up to it, and leaves for the
+  // level passes to finish (with subtrees, k_subtree takes all up to SUB_MAX)
+  bool run_big = false, run_small = !use_sub, run_leaf = true;
+  for (int64_t b = 0; b < nboxes; ++b) run_big = run_big || box_off_h[b + 1] - box_off_h[b] > CM_SMALL;
+  int64_t nsub = 0;
   for (;;) {
     int64_t lb = T.level_start[depth], le = T.level_start[depth + 1];
     int64_t nl = le - lb;
@@ -1738,7 +2261,14 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
     PartBlock *pb = dptr<PartBlock>(S.pblocks);
     HSR_HIP(dbuf_reserve(S.pnode, sizeof(int32_t) * pcap));
     int32_t *pnode = dptr<int32_t>(S.pnode);
-    k_part_plan<<<nblk_for(nl, 64), 64, 0, st>>>(nodes, lb, le, unit, cms, nd, c->p.ppc, unit_ppm, pnode, ctr);
+    k_part_plan<<<nblk_for(nl, 64), 64, 0, st>>>(nodes, lb, le, unit, cms, nd, c->p.ppc, unit_ppm, pnode, ctr,
+                                                 use_sub ? (depth == 0 ? 2 : cur) : -1);
+    if (use_sub && !run_big && depth > 0) {  // nothing but subtrees left
+      nsub += nl;
+      T.level_start.push_back(le);
+      ++depth;
+      continue;
+    }
     if (!unit_ppm && run_leaf) k_leaf_ppm<<<gnl, 64, 0, st>>>(nodes, lb, le, nd, Mr);
     if (run_leaf)
       k_finalize_leaves<<<(unsigned)nl, 64, 0, st>>>(nodes, lb, le, NODE_LEAF, depth == 0, P[cur], Pfin, unit,
@@ -1781,15 +2311,70 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
 #endif
     T.level_start.push_back(le + 2 * hc.nsplit);
     active = hc.active_next;
+    nsub += hc.nsub;
     run_big = hc.next_big > 0;
-    run_small = hc.next_small > 0;
-    run_leaf = hc.next_leaf > 0;
+    run_small = !use_sub && hc.next_small > 0;
+    run_leaf = hc.next_leaf > 0 && (!use_sub || nd > SUB_MAX);
     cur ^= 1;
     ++depth;
   }
   int nlev = (int)T.level_start.size() - 1;  // last level is empty
-  T.nnodes_bfs = T.level_start.back();
+  const int64_t upper = T.level_start.back();  // nodes of the level passes
+  T.nnodes_bfs = upper;
   T.max_depth = std::max(0, nlev - 2);  // deepest non-empty level index
+  if (nsub > 0) {
+    // ---- subtrees
+    HSR_HIP(dbuf_reserve(S.cnode, sizeof(int2) * (size_t)nsub + sizeof(int32_t) + 16));
+    int2 *list = dptr<int2>(S.cnode);
+    int32_t *count = reinterpret_cast<int32_t *>(list + nsub);
+    k_sub_init<<<1, 64, 0, st>>>(sub_ctr, upper, count);
+    k_sub_gather<<<nblk_for(upper, 256), 256, 0, st>>>(nodes, upper, list, count);
+    SubArrays A;
+    for (int k = 0; k < 2; ++k) {
+      A.x[k] = X[k];
+      A.y[k] = Y[k];
+      A.z[k] = Z[k];
+      A.p[k] = P[k];
+    }
+    A.x[2] = x;
+    A.y[2] = y;
+    A.z[2] = z;
+    // node slots: a few per leaf of nd / 2, more when a launch runs out
+    int64_t want = std::min<int64_t>(upper + 2 * n, upper + 5 * (n / nd) + 4 * nsub + 1024);
+    for (;;) {
+      if (want > cap) {
+        DBuf nbuf;
+        HSR_HIP(dbuf_reserve(nbuf, sizeof(BNode) * want));
+        HSR_HIP(hipMemcpyAsync(nbuf.p, T.bnodes.p, sizeof(BNode) * upper, hipMemcpyDeviceToDevice, st));
+        HSR_HIP(stream_wait(st));
+        dbuf_free(T.bnodes);
+        T.bnodes = nbuf;
+        cap = want;
+        nodes = dptr<BNode>(T.bnodes);
+      }
+      k_subtree<<<(unsigned)nsub, SUB_T, 0, st>>>(nodes, list, A, nd, c->p.ppc, cap, sub_ctr, Pfin, xs_, ys_,
+                                                  zs_, ms_);
+      HSR_HIP(hipGetLastError());
+      SubCtr hs;
+      HSR_HIP(hipMemcpyAsync(&hs, sub_ctr, sizeof(SubCtr), hipMemcpyDeviceToHost, st));
+      HSR_HIP(stream_wait(st));
+      if (hs.deep) {
+        *too_deep = true;
+        return HSR_OK;
+      }
+      if (!hs.overflow) {
+        T.nnodes_bfs = hs.next;
+        T.max_depth = std::max(T.max_depth, hs.depth);
+        break;
+      }
+      if (want >= upper + 2 * n) {
+        hsr_set_error("tree build: subtrees ran out of node slots");
+        return HSR_ERR_STATE;
+      }
+      want = std::min<int64_t>(upper + 2 * n, 2 * std::max(want, hs.next));
+      k_sub_init<<<1, 64, 0, st>>>(sub_ctr, upper, nullptr);
+    }
+  }
   int64_t nb = T.nnodes_bfs;
 
   // ---- bottom-up, top-down
@@ -1803,6 +2388,7 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
     int64_t lb = T.level_start[l], le = T.level_start[l + 1];
     if (le > lb) k_top_down<<<nblk_for(le - lb, 64), 64, 0, st>>>(nodes, lb, le);
   }
+  if (nb > upper) k_sub_top_down<<<nblk_for(nb - upper, 256), 256, 0, st>>>(nodes, upper, nb);
   // per-box canonical bases: box b holds 1 + 2 * sa(root_b) nodes
   std::vector<BNode> roots(nboxes);
   HSR_HIP(hipMemcpyAsync(roots.data(), nodes, sizeof(BNode) * nboxes, hipMemcpyDeviceToHost, st));
@@ -1839,11 +2425,10 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
     HSR_HIP(dbuf_reserve(T.ppm12, sizeof(float) * 12 * std::max<int64_t>(T.nnodes, 1)));
     float *ppm12 = dptr<float>(T.ppm12);
     if (T.nnodes > 0) k_zero_f32<<<nblk_for(12 * T.nnodes, 256), 256, 0, st>>>(12 * T.nnodes, ppm12);
-    for (int l = nlev - 1; l >= 0; --l) {
-      int64_t lb = T.level_start[l], le = T.level_start[l + 1];
-      if (le > lb)
-        k_pp12_level<<<nblk_for(12 * (le - lb), 256), 256, 0, st>>>(
-            nodes, lb, le, d_cbase, box_of, cn, dptr<float>(T.xs), dptr<float>(T.ys), dptr<float>(T.zs),
+    for (int64_t d = T.max_depth; d >= 0; --d) {
+      if (nb > 0)
+        k_pp12_level<<<nblk_for(12 * nb, 256), 256, 0, st>>>(
+            nodes, nb, (int)d, d_cbase, box_of, cn, dptr<float>(T.xs), dptr<float>(T.ys), dptr<float>(T.zs),
             dptr<float>(T.ms), ppm12);
     }
     if (T.nnodes > 0)
@@ -1853,4 +2438,14 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
   }
   HSR_HIP(hipGetLastError());
   return HSR_OK;
+}
+
+hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes, const int64_t *box_off, const float *min_loc,
+                             const float *max_loc, const float *x, const float *y, const float *z,
+                             const float *m) {
+  bool too_deep = false;
+  hsr_status s = build_levels(c, nboxes, box_off, min_loc, max_loc, x, y, z, m, true, &too_deep);
+  if (s == HSR_OK && too_deep)
+    s = build_levels(c, nboxes, box_off, min_loc, max_loc, x, y, z, m, false, &too_deep);
+  return s;
 }
