@@ -475,6 +475,18 @@ __global__ void k_item_count(int64_t nleaves, const int64_t *ent_ptr,
   psize[k] = c > 1 ? c * 3 * cn[leaves[k]].count : 0;
 }
 
+// The plan's totals: items, leaves with several, partial floats; the counts
+// the force phase reads are its first two.
+__global__ void k_plan_totals(int64_t nl, const int64_t *item_base, const int64_t *nitem,
+                              const int64_t *mpos, const int64_t *mflag, const int64_t *pbase,
+                              const int64_t *psize, int64_t *counts) {
+  if (threadIdx.x == 0) {
+    counts[0] = item_base[nl - 1] + nitem[nl - 1];
+    counts[1] = mpos[nl - 1] + mflag[nl - 1];
+    counts[2] = pbase[nl - 1] + psize[nl - 1];
+  }
+}
+
 // Work classes of the queue, heaviest first: four to the octave.
 constexpr int NCLASS = 256;
 
@@ -835,7 +847,7 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   }
   // scratch layout (int64 unless noted), arrays at a stride that only grows,
   // so their addresses (held by a captured force phase) survive list builds
-  if (nl + 1 > LS.plan_stride) LS.plan_stride = std::max<int64_t>(nl + 1, LS.plan_stride + LS.plan_stride / 4);
+  if (nl + 3 > LS.plan_stride) LS.plan_stride = std::max<int64_t>(nl + 3, LS.plan_stride + LS.plan_stride / 4);
   const int64_t ps = LS.plan_stride;
   HSR_HIP(dbuf_reserve(LS.plan, sizeof(int64_t) * 8 * ps + sizeof(int32_t) * ps + 256));
   int64_t *nitem = dptr<int64_t>(LS.plan);
@@ -855,17 +867,12 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   if ((s = excl_scan(c, nitem, item_base, nl)) != HSR_OK) return s;
   if ((s = excl_scan(c, mflag, mpos, nl)) != HSR_OK) return s;
   if ((s = excl_scan(c, psize, pbase, nl)) != HSR_OK) return s;
-  int64_t tail[6];
-  HSR_HIP(hipMemcpyAsync(&tail[0], item_base + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&tail[1], nitem + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&tail[2], mpos + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&tail[3], mflag + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&tail[4], pbase + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&tail[5], psize + nl - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  // (the arrays' stride leaves counts room for its three words)
+  k_plan_totals<<<1, 64, 0, st>>>(nl, item_base, nitem, mpos, mflag, pbase, psize, counts);
+  int64_t tail[3];
+  HSR_HIP(hipMemcpyAsync(tail, counts, sizeof(tail), hipMemcpyDeviceToHost, st));
   HSR_HIP(stream_wait(st));
-  const int64_t nitems = tail[0] + tail[1];
-  const int64_t nmulti = tail[2] + tail[3];
-  const int64_t npart = tail[4] + tail[5];
+  const int64_t nitems = tail[0], nmulti = tail[1], npart = tail[2];
   // the item ids are 32-bit
   if (nitems >= (int64_t)INT32_MAX) {
     hsr_set_error("force plan: " + std::to_string(nitems) +
@@ -891,10 +898,6 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
                                              items_tmp, hist, multi, mpos, mflag);
   // heaviest items first
   k_item_order<<<nblk(nitems, 256), 256, 0, st>>>(nitems, items_tmp, hist, hist + NCLASS, items);
-  // device-resident counts for the persistent launch
-  int64_t hc[2] = {nitems, nmulti};
-  HSR_HIP(hipMemcpyAsync(counts, hc, sizeof(hc), hipMemcpyHostToDevice, st));
-  HSR_HIP(stream_wait(st));
   LS.multi = multi;
   LS.counts = counts;
   LS.leaf_pbase = pbase;

@@ -120,6 +120,7 @@ struct TreeState {
   bool unit = false;          // every mass of the last build was exactly 1.0f
   int64_t nboxes = 1;
   std::vector<int64_t> box_root;  // BFS id of each box root
+  std::vector<int64_t> box_leaves;  // visited leaves of each box
 };
 
 struct ListState {

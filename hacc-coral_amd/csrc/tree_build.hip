@@ -2394,7 +2394,11 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
   HSR_HIP(hipMemcpyAsync(roots.data(), nodes, sizeof(BNode) * nboxes, hipMemcpyDeviceToHost, st));
   HSR_HIP(stream_wait(st));
   std::vector<int64_t> cbase(nboxes + 1, 0);
-  for (int64_t b = 0; b < nboxes; ++b) cbase[b + 1] = cbase[b] + 1 + 2 * roots[b].sa;
+  T.box_leaves.resize(nboxes);
+  for (int64_t b = 0; b < nboxes; ++b) {
+    cbase[b + 1] = cbase[b] + 1 + 2 * roots[b].sa;
+    T.box_leaves[b] = roots[b].nleaf;
+  }
   T.nnodes = cbase[nboxes];
   T.box_root.assign(cbase.begin(), cbase.end());
   HSR_HIP(dbuf_reserve(S.e, sizeof(int64_t) * (nboxes + 1) + sizeof(int32_t) * (nb + nboxes) + 64));
