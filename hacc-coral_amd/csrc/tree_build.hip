@@ -1359,9 +1359,7 @@ __global__ void k_bottom_up(BNode *nodes, int64_t lb, int64_t le, float ppc,
 
 // Top-down: canonical ids (children get 1 + 2A and 2 + 2A, A = allocating
 // nodes before the parent in preorder) and the right-first leaf rank.
-__global__ void k_top_down(BNode *nodes, int64_t lb, int64_t le) {
-  int64_t t = lb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= le) return;
+__device__ __forceinline__ void top_down_node(BNode *nodes, int64_t t) {
   BNode &n = nodes[t];
   if (n.kind != NODE_SPLIT) return;
   BNode &L = nodes[n.cl];
@@ -1372,6 +1370,39 @@ __global__ void k_top_down(BNode *nodes, int64_t lb, int64_t le) {
   R.canon = 2 + 2 * n.a;
   R.leaf_rank = n.leaf_rank;
   L.leaf_rank = n.leaf_rank + R.nleaf;
+}
+
+__global__ void k_top_down(BNode *nodes, int64_t lb, int64_t le) {
+  int64_t t = lb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t < le) top_down_node(nodes, t);
+}
+
+// A run of consecutive levels of at most RUN_NODES nodes each by one
+// workgroup, a barrier between levels: a launch a level costs such levels
+// more than their work (4 to 5 us; here about 2).
+constexpr int RUN_NODES = 1024, RUN_LEVELS = 32;
+struct LevelRun {
+  int n;
+  int64_t start[RUN_LEVELS + 1];
+};
+
+__global__ void __launch_bounds__(RUN_NODES)
+k_bottom_up_run(BNode *nodes, LevelRun R, float ppc, const int32_t *Pfin, const float *Min) {
+  for (int v = R.n - 1; v >= 0; --v) {
+    const int64_t t = R.start[v] + threadIdx.x;
+    if (t < R.start[v + 1]) bottom_up_node(nodes, t, ppc, Pfin, Min);
+    __threadfence_block();
+    __syncthreads();
+  }
+}
+
+__global__ void __launch_bounds__(RUN_NODES) k_top_down_run(BNode *nodes, LevelRun R) {
+  for (int v = 0; v < R.n; ++v) {
+    const int64_t t = R.start[v] + threadIdx.x;
+    if (t < R.start[v + 1]) top_down_node(nodes, t);
+    __threadfence_block();
+    __syncthreads();
+  }
 }
 
 __global__ void k_write_canon(const BNode *nodes, int64_t nb,
@@ -1413,14 +1444,13 @@ __global__ void k_write_canon(const BNode *nodes, int64_t nb,
   }
 }
 
-__global__ void k_box_of(const BNode *nodes, int64_t nb, int32_t *box_of,
-                         const int32_t *root_box) {
-  // root_box[t] = box of root t or -1; walk parents
+__global__ void k_box_of(const BNode *nodes, int64_t nb, int32_t *box_of) {
+  // the roots are the first nodes, in box order; walk parents
   int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (t >= nb) return;
   int64_t u = t;
   while (nodes[u].parent >= 0) u = nodes[u].parent;
-  box_of[t] = root_box[u];
+  box_of[t] = (int32_t)u;
 }
 
 // ------------------------------------------------------------ subtrees
@@ -2379,14 +2409,35 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
 
   // ---- bottom-up, top-down
   const float *Min = m;
-  for (int l = nlev - 1; l >= 0; --l) {
-    int64_t lb = T.level_start[l], le = T.level_start[l + 1];
-    if (le > lb)
+  // levels [l0, l1) of at most RUN_NODES nodes each, as a run
+  auto level_run = [&](int l0, int l1) {
+    LevelRun R;
+    R.n = l1 - l0;
+    for (int l = l0; l <= l1; ++l) R.start[l - l0] = T.level_start[l];
+    return R;
+  };
+  auto small = [&](int l) { return T.level_start[l + 1] - T.level_start[l] <= RUN_NODES; };
+  for (int l = nlev; l > 0;) {
+    int l0 = l - 1;
+    if (small(l0)) {
+      while (l0 > 0 && l - l0 < RUN_LEVELS && small(l0 - 1)) --l0;
+      k_bottom_up_run<<<1, RUN_NODES, 0, st>>>(nodes, level_run(l0, l), c->p.ppc, Pfin, Min);
+    } else {
+      const int64_t lb = T.level_start[l0], le = T.level_start[l];
       k_bottom_up<<<nblk_for(le - lb, 64), 64, 0, st>>>(nodes, lb, le, c->p.ppc, Pfin, Min);
+    }
+    l = l0;
   }
-  for (int l = 0; l < nlev; ++l) {
-    int64_t lb = T.level_start[l], le = T.level_start[l + 1];
-    if (le > lb) k_top_down<<<nblk_for(le - lb, 64), 64, 0, st>>>(nodes, lb, le);
+  for (int l = 0; l < nlev;) {
+    int l1 = l + 1;
+    if (small(l)) {
+      while (l1 < nlev && l1 - l < RUN_LEVELS && small(l1)) ++l1;
+      k_top_down_run<<<1, RUN_NODES, 0, st>>>(nodes, level_run(l, l1));
+    } else {
+      const int64_t lb = T.level_start[l], le = T.level_start[l1];
+      k_top_down<<<nblk_for(le - lb, 64), 64, 0, st>>>(nodes, lb, le);
+    }
+    l = l1;
   }
   if (nb > upper) k_sub_top_down<<<nblk_for(nb - upper, 256), 256, 0, st>>>(nodes, upper, nb);
   // per-box canonical bases: box b holds 1 + 2 * sa(root_b) nodes
@@ -2401,19 +2452,13 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
   }
   T.nnodes = cbase[nboxes];
   T.box_root.assign(cbase.begin(), cbase.end());
-  HSR_HIP(dbuf_reserve(S.e, sizeof(int64_t) * (nboxes + 1) + sizeof(int32_t) * (nb + nboxes) + 64));
+  HSR_HIP(dbuf_reserve(S.e, sizeof(int64_t) * (nboxes + 1) + 64));
   int64_t *d_cbase = dptr<int64_t>(S.e);
-  int32_t *root_box = reinterpret_cast<int32_t *>(d_cbase + nboxes + 1);
-  HSR_HIP(hipMemcpyAsync(d_cbase, cbase.data(), sizeof(int64_t) * (nboxes + 1), hipMemcpyHostToDevice, st));
-  {
-    std::vector<int32_t> rb(nboxes);
-    for (int64_t b = 0; b < nboxes; ++b) rb[b] = (int32_t)b;
-    HSR_HIP(hipMemcpyAsync(root_box, rb.data(), sizeof(int32_t) * nboxes, hipMemcpyHostToDevice, st));
-    HSR_HIP(stream_wait(st));
-  }
+  // (from the context's copy, which outlives the call)
+  HSR_HIP(hipMemcpyAsync(d_cbase, T.box_root.data(), sizeof(int64_t) * (nboxes + 1), hipMemcpyHostToDevice, st));
   HSR_HIP(dbuf_reserve(S.f, sizeof(int32_t) * (nb + 1)));
   int32_t *box_of = dptr<int32_t>(S.f);
-  k_box_of<<<nblk_for(nb, 256), 256, 0, st>>>(nodes, nb, box_of, root_box);
+  k_box_of<<<nblk_for(nb, 256), 256, 0, st>>>(nodes, nb, box_of);
   HSR_HIP(dbuf_reserve(T.canon_nodes, sizeof(hsr_node) * std::max<int64_t>(T.nnodes, 1)));
   hsr_node *cn = dptr<hsr_node>(T.canon_nodes);
   k_write_canon<<<nblk_for(nb, 256), 256, 0, st>>>(nodes, nb, d_cbase, box_of, cn);
