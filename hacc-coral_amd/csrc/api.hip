@@ -346,6 +346,87 @@ hsr_status stage_out(hsr_ctx *c, int64_t n, float *const f[8], int64_t *id, uint
 
 void hsr_set_error(const std::string &msg) { g_err = msg; }
 
+namespace {
+
+// Buffers of destroyed contexts, kept for the next ones.  The reference's
+// surface makes a tree object a step (RCBForceTree's constructor does all the
+// work), so a drop-in caller creates and destroys a context a step, and the
+// runtime's allocations and frees of its forty buffers cost 1.6 ms to give
+// back and half as much to get (a 48^3 step through the constructor: 6.2 ms,
+// 4.1 with the buffers kept).
+// Bounded: at most KEEP_BYTES a device, none above KEEP_ONE, the oldest
+// freed first; all are given back when an allocation fails.  A buffer enters
+// only after its context's stream has been waited for (hsr_destroy), so the
+// next owner may use it on any stream.
+constexpr size_t KEEP_BYTES = (size_t)1 << 30, KEEP_ONE = (size_t)1 << 28;
+struct Kept {
+  void *p;
+  size_t bytes;
+  int device;
+};
+std::mutex g_kept_mutex;
+std::vector<Kept> g_kept;  // oldest first
+
+// The smallest kept buffer of the current device that holds `bytes` and is
+// not much larger; null if there is none.
+void *kept_take(size_t bytes, size_t *got) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(g_kept_mutex);
+  size_t best = g_kept.size();
+  for (size_t i = 0; i < g_kept.size(); ++i)
+    if (g_kept[i].device == dev && g_kept[i].bytes >= bytes && g_kept[i].bytes <= 2 * bytes + 65536 &&
+        (best == g_kept.size() || g_kept[i].bytes < g_kept[best].bytes))
+      best = i;
+  if (best == g_kept.size()) return nullptr;
+  void *p = g_kept[best].p;
+  *got = g_kept[best].bytes;
+  g_kept.erase(g_kept.begin() + (ptrdiff_t)best);
+  return p;
+}
+
+// Keeps an idle buffer of the current device, or frees it.
+void kept_put(void *p, size_t bytes) {
+  int dev = 0;
+  if (bytes > KEEP_ONE || hipGetDevice(&dev) != hipSuccess) {
+    (void)hipFree(p);
+    return;
+  }
+  std::lock_guard<std::mutex> lock(g_kept_mutex);
+  g_kept.push_back({p, bytes, dev});
+  size_t total = 0;
+  for (const Kept &k : g_kept) total += k.device == dev ? k.bytes : 0;
+  for (size_t i = 0; total > KEEP_BYTES && i < g_kept.size();) {
+    if (g_kept[i].device != dev) {
+      ++i;
+      continue;
+    }
+    total -= g_kept[i].bytes;
+    (void)hipFree(g_kept[i].p);
+    g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
+  }
+}
+
+// Gives every kept buffer of the current device back; whether there was one.
+bool kept_release() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_kept_mutex);
+  bool any = false;
+  for (size_t i = 0; i < g_kept.size();) {
+    if (g_kept[i].device != dev) {
+      ++i;
+      continue;
+    }
+    (void)hipFree(g_kept[i].p);
+    g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
+    any = true;
+  }
+  return any;
+}
+
+}  // namespace
+
 hipError_t dbuf_reserve(DBuf &b, size_t bytes) {
   if (bytes <= b.bytes && b.p) return hipSuccess;
   // a buffer that grows again takes a quarter more than asked, so slowly
@@ -359,10 +440,19 @@ hipError_t dbuf_reserve(DBuf &b, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
   }
+  b.p = kept_take(want, &want);
+  if (b.p) {
+    b.bytes = want;
+    return hipSuccess;
+  }
   hipError_t e = hipMalloc(&b.p, want);
   if (e != hipSuccess && want > bytes) {  // no room for the slack: the size asked
     (void)hipGetLastError();
     want = std::max<size_t>(bytes, 256);
+    e = hipMalloc(&b.p, want);
+  }
+  if (e != hipSuccess && kept_release()) {  // no room beside the kept buffers
+    (void)hipGetLastError();
     e = hipMalloc(&b.p, want);
   }
   if (e != hipSuccess) {
@@ -489,7 +579,7 @@ hsr_status hsr_destroy(hsr_ctx *c) {
   DBuf *bufs[] = {&c->tree.bnodes, &c->tree.canon_nodes, &c->tree.pfin, &c->tree.pj, &c->tree.ppm12,
                   &c->tree.xs, &c->tree.ys, &c->tree.zs, &c->tree.ms,
                   &c->lists.leaves, &c->lists.seg_ptr, &c->lists.seg, &c->lists.ent_ptr,
-                  &c->lists.jidx, &c->lists.items, &c->lists.segcache,
+                  &c->lists.jidx, &c->lists.iperm, &c->lists.items, &c->lists.segcache,
                   &c->lists.item_keys,
                   &c->lists.plan, &c->lists.part, &c->s.qctr,
                   &c->adj.fw, &c->adj.fw_items, &c->adj.tr, &c->adj.tr_items, &c->adj.seg,
@@ -501,14 +591,19 @@ hsr_status hsr_destroy(hsr_ctx *c) {
                   &c->s.pblocks, &c->s.cnode, &c->s.pnode, &c->s.pmask, &c->s.counters, &c->dev_v, &c->force};
   if (c->adj.graph_exec) (void)hipGraphExecDestroy(c->adj.graph_exec);
   if (c->adj.graph) (void)hipGraphDestroy(c->adj.graph);
-  for (DBuf *b : bufs) dbuf_free(*b);
-  for (int k = 0; k < 10; ++k) dbuf_free(c->s.host_in[k]);
-  dbuf_free(c->sub.keys);
-  dbuf_free(c->sub.stage);
-  dbuf_free(c->sub.xcnt);
-  dbuf_free(c->sub.xstage);
-  dbuf_free(c->sub.xout);
-  for (int k = 0; k < 10; ++k) dbuf_free(c->sub.arr[k]);
+  auto give = [](DBuf &b) {  // idle: the stream has been waited for
+    if (b.p) kept_put(b.p, b.bytes);
+    b.p = nullptr;
+    b.bytes = 0;
+  };
+  for (DBuf *b : bufs) give(*b);
+  for (int k = 0; k < 10; ++k) give(c->s.host_in[k]);
+  give(c->sub.keys);
+  give(c->sub.stage);
+  give(c->sub.xcnt);
+  give(c->sub.xstage);
+  give(c->sub.xout);
+  for (int k = 0; k < 10; ++k) give(c->sub.arr[k]);
   for (int k = 0; k < 6; ++k)
     if (c->sub.ev[k]) (void)hipEventDestroy(c->sub.ev[k]);
   for (int k = 0; k < 8; ++k) (void)hipEventDestroy(c->ev[k]);
