@@ -711,7 +711,8 @@ LawArgs law_args(const ForceLawDev &D) {
 }  // namespace
 
 // Target order inside each listed leaf: positions sorted along the leaf's
-// longest box edge (ties x > y > z; equal coordinates by position), so that
+// longest box edge (ties x > y > z; coordinates equal in their leading
+// 22 bits by position), so that
 // a pass's 128 targets span a slab of the leaf and the entries its box is
 // beyond the cutoff of can be skipped.  iperm[off + k] = position of the
 // k-th target; leaves above SORT_MAX keep their order.
@@ -722,53 +723,39 @@ __global__ void k_iota32(int64_t n, int32_t *a) {
   if (k < n) a[k] = (int32_t)k;
 }
 
+// Every target's place is the number of smaller keys in its leaf: n broadcast
+// LDS reads a target and no barriers, where a bitonic sort took log^2 n of
+// them (0.68 -> 0.41 ms at 256^3 with leaves of 512).  The keys are the
+// coordinate's leading 22 bits, then the position, so no two are equal; the
+// passes need no finer order.
 __global__ void __launch_bounds__(256)
 k_leaf_sort(int64_t nl, const int32_t *__restrict__ leaves, const hsr_node *__restrict__ cn,
             const PJ *__restrict__ pj, int32_t *__restrict__ iperm) {
-  __shared__ float key[SORT_MAX];
-  __shared__ int32_t idx[SORT_MAX];
+  __shared__ uint32_t key[SORT_MAX];
   const int64_t k = blockIdx.x;
   if (k >= nl) return;
   const hsr_node &nd = cn[leaves[k]];
-  const int64_t off = nd.offset, cnt = nd.count;
-  if (cnt < 2 || cnt > SORT_MAX) return;
+  const int64_t off = nd.offset;
+  if (nd.count < 2 || nd.count > SORT_MAX) return;
+  const int cnt = (int)nd.count;
   const float e0 = nd.xmax[0] - nd.xmin[0], e1 = nd.xmax[1] - nd.xmin[1],
               e2 = nd.xmax[2] - nd.xmin[2];
   const int d = (e0 >= e1 && e0 >= e2) ? 0 : (e1 >= e2 ? 1 : 2);
-  int np2 = 2;
-  while (np2 < cnt) np2 <<= 1;
-  for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-    if (i < cnt) {
-      const PJ p = pj[off + i];
-      key[i] = d == 0 ? p.x : (d == 1 ? p.y : p.z);
-    } else {
-      key[i] = INFINITY;
-    }
-    idx[i] = i;
+  for (int i = threadIdx.x; i < cnt; i += 256) {
+    const PJ p = pj[off + i];
+    const uint32_t u = __float_as_uint(d == 0 ? p.x : (d == 1 ? p.y : p.z));
+    // an unsigned number in the order of the floats
+    const uint32_t ord = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+    key[i] = (ord & ~(uint32_t)(SORT_MAX - 1)) | (uint32_t)i;
   }
   __syncthreads();
-  // bitonic sort of (key, idx), ascending and lexicographic
-  for (int size = 2; size <= np2; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-        const int j = i ^ stride;
-        if (j > i) {
-          const bool up = (i & size) == 0;
-          const float ki = key[i], kj = key[j];
-          const int32_t ii = idx[i], ij = idx[j];
-          const bool gt = ki > kj || (ki == kj && ii > ij);
-          if (gt == up) {
-            key[i] = kj;
-            key[j] = ki;
-            idx[i] = ij;
-            idx[j] = ii;
-          }
-        }
-      }
-      __syncthreads();
-    }
+  for (int i = threadIdx.x; i < cnt; i += 256) {
+    const uint32_t mine = key[i];
+    int rank = 0;
+#pragma unroll 8
+    for (int q = 0; q < cnt; ++q) rank += key[q] < mine ? 1 : 0;
+    iperm[off + rank] = (int32_t)(off + i);
   }
-  for (int i = threadIdx.x; i < cnt; i += blockDim.x) iperm[off + i] = (int32_t)(off + idx[i]);
 }
 
 // Shapes built for every polynomial law without the r2 > 0 guard (the
