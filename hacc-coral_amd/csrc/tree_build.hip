@@ -307,19 +307,27 @@ k_cm_plan(BNode *nodes, int64_t lb, int64_t le, int32_t *cnode, Counters *ctr) {
   }
 }
 
-// Approximate sums and bbox per block (one wave per block).  With unit
+// Approximate sums and bbox per block by NW waves (each a run of CM_BLK / NW
+// elements; the first merges them).  One wave is a chain of some 1500
+// instructions, which sets the level's time where the chip's SIMDs outnumber
+// the blocks: four waves a block there (14.2 -> 9.8 us a level at 365k
+// particles; with 2400 blocks 17.8 -> 18.7, so one wave from there on).  With unit
 // masses (UNIT) the mass sum's record is written directly: approximate sum
 // and integer sum len in units of 2^0.  The block's integer sum of a
 // nonnegative sum is taken in units of its finest lsb (LaneSum); one that
 // reaches 2^53 units is marked as not an integer there, which leaves its
 // node off the integer path just as the node's total would.
-template <bool UNIT>
-__global__ void __launch_bounds__(64)
+template <bool UNIT, int NW>
+__global__ void __launch_bounds__(64 * NW)
 k_cm_blk_stats(const BNode *nodes, const int32_t *cnode, CmBlock *blk, const Counters *ctr,
                const float *X, const float *Y, const float *Z, const float *M) {
   constexpr int NQ = UNIT ? 3 : 4;  // sums formed from the addends
   constexpr int RU = 4;             // elements per lane per load round
-  const int l = lane_id();
+  constexpr int RUN = CM_PER / NW;  // elements per lane
+  __shared__ float psum[NW][4], pmn[NW][3], pmx[NW][3];
+  __shared__ uint64_t pun[NW][4];
+  __shared__ int32_t plsb[NW][4], pflag[NW][4];
+  const int l = lane_id(), w = threadIdx.x >> 6;
   for (int64_t b = blockIdx.x; b < ctr->cm_blocks; b += gridDim.x) {
     CmBlock &B = blk[b];
     int64_t start;
@@ -333,7 +341,7 @@ k_cm_blk_stats(const BNode *nodes, const int32_t *cnode, CmBlock *blk, const Cou
     // rounds of RU elements per lane: the loads of a round are in flight
     // together and few values stay live
 #pragma unroll 1
-    for (int i0 = 0; i0 < CM_PER; i0 += RU) {
+    for (int i0 = w * RUN; i0 < (w + 1) * RUN; i0 += RU) {
       float xv[RU], yv[RU], zv[RU], wv[RU];
 #pragma unroll
       for (int i = 0; i < RU; ++i) {
@@ -383,6 +391,43 @@ k_cm_blk_stats(const BNode *nodes, const int32_t *cnode, CmBlock *blk, const Cou
     for (int d = 0; d < 3; ++d) {
       mn[d] = wave_min_f32(mn[d]);
       mx[d] = wave_max_f32(mx[d]);
+    }
+    if (NW > 1) {
+      __syncthreads();  // the previous block's records have been merged
+      if (l == 0) {
+        for (int q = 0; q < NQ; ++q) {
+          psum[w][q] = s[q];
+          pun[w][q] = un[q];
+          plsb[w][q] = lsb[q];
+          pflag[w][q] = bad[q];
+        }
+        for (int d = 0; d < 3; ++d) {
+          pmn[w][d] = mn[d];
+          pmx[w][d] = mx[d];
+        }
+      }
+      __syncthreads();
+      if (w != 0) continue;
+      // lanes below NW hold a run each: the merge is the wave's again
+      const bool v = l < NW;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        s[q] = wave_sum_f32(v ? psum[v ? l : 0][q] : 0.f);
+        const int32_t lq = v ? plsb[v ? l : 0][q] : (1 << 20);
+        const bool neg_q = __any(lq == INT32_MIN);
+        LaneSum r;
+        r.u = v ? pun[v ? l : 0][q] : 0ull;
+        r.t = lq == INT32_MIN ? (1 << 20) : lq;
+        r.bad = v && pflag[v ? l : 0][q];
+        if (r.bad) r.u = 0;
+        un[q] = wave_lane_sum(r, lsb[q], bad[q]);
+        if (neg_q) lsb[q] = INT32_MIN;
+      }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        mn[d] = wave_min_f32(v ? pmn[v ? l : 0][d] : INFINITY);
+        mx[d] = wave_max_f32(v ? pmx[v ? l : 0][d] : -INFINITY);
+      }
     }
     if (l == 0) {
       for (int q = 0; q < 4; ++q) {
@@ -2271,10 +2316,14 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
       k_cm_plan<<<nblk_for(nl, 64), 64, 0, st>>>(nodes, lb, le, cnode, ctr);
       unsigned cmg = (unsigned)std::max<int64_t>(1, active / CM_BLK + active / CM_SMALL + 1);
       cmg = std::min(cmg, gbig);
-      if (unit)
-        k_cm_blk_stats<true><<<cmg, 64, 0, st>>>(nodes, cnode, cmb, ctr, Xr, Yr, Zr, Mr);
-      else
-        k_cm_blk_stats<false><<<cmg, 64, 0, st>>>(nodes, cnode, cmb, ctr, Xr, Yr, Zr, Mr);
+      const bool few = cm_cap <= (int64_t)std::max(1, c->num_cus) * 4;
+#define BLK_STATS(UNIT, NW) \
+  k_cm_blk_stats<UNIT, NW><<<cmg, 64 * NW, 0, st>>>(nodes, cnode, cmb, ctr, Xr, Yr, Zr, Mr)
+      if (unit && few) BLK_STATS(true, 4);
+      else if (unit) BLK_STATS(true, 1);
+      else if (few) BLK_STATS(false, 4);
+      else BLK_STATS(false, 1);
+#undef BLK_STATS
       const unsigned cmr = std::max(1u, std::min<unsigned>(gbig, (unsigned)(cm_cap / 64 + 1)));
       k_cm_chunk<<<cmr, 64, 0, st>>>(nodes, cnode, cmb, ctr);
       k_cm_node<<<gnl, 64, 0, st>>>(nodes, lb, le, cmb, cmflags, cms);
