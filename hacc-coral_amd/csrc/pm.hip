@@ -122,17 +122,33 @@ struct PMap {
 };
 constexpr int PMAP_SAT = 1 << 26;
 
-__device__ __forceinline__ int pmap_add(int a, int b) {
-  const long long s = (long long)a + b;
-  return s > PMAP_SAT ? PMAP_SAT : (int)s;
-}
-
-// a, then b
+// a, then b.  Both are in [0, PMAP_SAT]: their sum fits an int and
+// saturates with either.
 __device__ __forceinline__ PMap pmap_compose(PMap a, PMap b) {
   PMap m;
-  m.d0 = a.d0 >= PMAP_SAT ? PMAP_SAT : pmap_add(a.d0, (a.d0 & 1) ? b.d1 : b.d0);
-  m.d1 = a.d1 >= PMAP_SAT ? PMAP_SAT : pmap_add(a.d1, ((a.d1 + 1) & 1) ? b.d1 : b.d0);
+  m.d0 = min(a.d0 + ((a.d0 & 1) ? b.d1 : b.d0), PMAP_SAT);
+  m.d1 = min(a.d1 + ((a.d1 & 1) ? b.d0 : b.d1), PMAP_SAT);
   return m;
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ PMap pmap_dpp_step(PMap mp) {
+  PMap pv;  // lanes without a source, and rows left out, get the identity
+  pv.d0 = __builtin_amdgcn_update_dpp(0, mp.d0, CTRL, ROWS, 0xf, false);
+  pv.d1 = __builtin_amdgcn_update_dpp(0, mp.d1, CTRL, ROWS, 0xf, false);
+  return pmap_compose(pv, mp);
+}
+
+// Inclusive scan over a wave's lanes, all of them active: shifts within rows
+// of 16, then the rows' totals passed on (lane moves in the vector pipe
+// instead of 12 LDS permutes in a dependent chain).
+__device__ __forceinline__ PMap pmap_scan(PMap mp) {
+  mp = pmap_dpp_step<0x111, 0xf>(mp);  // row_shr 1, 2, 4, 8
+  mp = pmap_dpp_step<0x112, 0xf>(mp);
+  mp = pmap_dpp_step<0x114, 0xf>(mp);
+  mp = pmap_dpp_step<0x118, 0xf>(mp);
+  mp = pmap_dpp_step<0x142, 0xa>(mp);  // row_bcast 15 into rows 1 and 3
+  return pmap_dpp_step<0x143, 0xc>(mp);  // row_bcast 31 into rows 2 and 3
 }
 
 __device__ __forceinline__ PMap pmap_term(double t, int E) {
@@ -162,11 +178,16 @@ __device__ __forceinline__ PMap pmap_term(double t, int E) {
 // terms are added in order, reading them with v_readlane.  r is the same in
 // every lane.
 constexpr int LT = 4;
+constexpr int WAVE_HEAD = 32;
 
 __device__ __forceinline__ double pick(const double (&t)[LT], int k) {
   return k == 0 ? t[0] : k == 1 ? t[1] : k == 2 ? t[2] : t[3];
 }
 
+// HEAD: the sum starts here, and its first terms, where it leaves a binade
+// every few of them, are added directly (a pass of the scan costs about as
+// much as 32 additions).
+template <bool HEAD>
 __device__ __forceinline__ float wave_add_step(float r, const double (&t)[LT], int cnt) {
   static_assert(LT == 4, "pick() reads four terms per lane");
   const int l = threadIdx.x & 63;
@@ -181,6 +202,11 @@ __device__ __forceinline__ float wave_add_step(float r, const double (&t)[LT], i
     return r;
   }
   int s = 0;
+  if constexpr (HEAD) {
+#pragma unroll
+    for (int i = 0; i < WAVE_HEAD; ++i) r = cic_add(r, readlane_f64(t[i % LT], i / LT));  // zeros past cnt
+    s = WAVE_HEAD;
+  }
   while (s < cnt) {
     if (!(r >= 0x1p-125f)) {  // zero or subnormal: the double sum's grid varies
       r = cic_add(r, readlane_f64(pick(t, s % LT), s / LT));
@@ -196,13 +222,7 @@ __device__ __forceinline__ float wave_add_step(float r, const double (&t)[LT], i
       const int i = LT * l + k;
       if (i >= s && i < cnt) mp = pmap_compose(mp, pmap_term(t[k], E));
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      PMap pv;
-      pv.d0 = __shfl_up(mp.d0, off);
-      pv.d1 = __shfl_up(mp.d1, off);
-      if (l >= off) mp = pmap_compose(pv, mp);
-    }
+    mp = pmap_scan(mp);
     const int d = (R & 1) ? mp.d1 : mp.d0;
     const int Rl = d >= PMAP_SAT ? PMAP_SAT : R + d;
     // R only grows: the lanes past the crossing one cross too
@@ -291,13 +311,7 @@ k_cic_tail(int64_t m, const uint32_t *__restrict__ key, const double *__restrict
         const int i = LT * tid + k;
         if (i >= s && i < cnt) mp = pmap_compose(mp, pmap_term(t[k], E));
       }
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        PMap pv;
-        pv.d0 = __shfl_up(mp.d0, off);
-        pv.d1 = __shfl_up(mp.d1, off);
-        if (l >= off) mp = pmap_compose(pv, mp);
-      }
+      mp = pmap_scan(mp);
       if (l == 63) wtot[w] = mp;
       if (tid == 0) j_sh = TAIL_THREADS;
       __syncthreads();
@@ -395,17 +409,26 @@ __device__ __forceinline__ void weights(float xx, float yy, float zz, float &ab,
 __global__ void __launch_bounds__(256)
 k_cic_base(int64_t n, const float *__restrict__ x, const float *__restrict__ y,
            const float *__restrict__ z, Grid g, Ext ex, uint32_t *__restrict__ key,
-           int32_t *__restrict__ idx, int32_t *__restrict__ nout) {
+           int32_t *__restrict__ idx, int32_t *__restrict__ nout, int32_t *__restrict__ unsorted) {
   const int64_t nn = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (nn >= n) return;
+  auto base_key = [&](float xx, float yy, float zz) {
+    const int ix = x86_floor_int(xx), iy = x86_floor_int(yy), iz = x86_floor_int(zz);
+    const bool in = ix >= -1 && ix < g.ng0 && iy >= -1 && iy < g.ng1 && iz >= -1 && iz < g.ng2;
+    return in ? (((uint32_t)(ix + 1) * ex.e1 + (uint32_t)(iy + 1)) * ex.e2 + (uint32_t)(iz + 1)) : ex.out;
+  };
   const float xx = x[nn], yy = y[nn], zz = z[nn];
   const Corners cc = corners(xx, yy, zz, g);
   int no = 0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) no += cc.cell[q] == g.safe;
-  const int ix = x86_floor_int(xx), iy = x86_floor_int(yy), iz = x86_floor_int(zz);
-  const bool in = ix >= -1 && ix < g.ng0 && iy >= -1 && iy < g.ng1 && iz >= -1 && iz < g.ng2;
-  key[nn] = in ? (((uint32_t)(ix + 1) * ex.e1 + (uint32_t)(iy + 1)) * ex.e2 + (uint32_t)(iz + 1)) : ex.out;
+  const uint32_t k = base_key(xx, yy, zz);
+  // whether the keys are in order already: the lane before's, or for a
+  // wave's first lane the particle before's
+  uint32_t prev = (uint32_t)__shfl_up((int)k, 1);
+  if ((threadIdx.x & 63) == 0) prev = nn > 0 ? base_key(x[nn - 1], y[nn - 1], z[nn - 1]) : 0u;
+  if (prev > k) unsorted[0] = 1;  // every writer stores the same value
+  key[nn] = k;
   idx[nn] = (int32_t)nn;
   nout[nn] = no;
 }
@@ -461,8 +484,19 @@ __device__ __forceinline__ void merge_advance(int qs, int32_t (&s)[8], const int
     }
 }
 
+// The corners in the order of their base cells' keys, for any cell: with the
+// particles in base-cell order (k_cic_base) a cell's contributions are its
+// eight lists one after another in this order.
+constexpr int kCornerByKey[8] = {5, 6, 4, 7, 2, 1, 3, 0};
+__constant__ int kCornerByKeyDev[8] = {5, 6, 4, 7, 2, 1, 3, 0};
+
 // One thread per grid cell: at most CELL_SHORT contributions are merged and
 // added here; longer cells are queued with their counts for k_cic_long_sum.
+// INORDER: the particles are in base-cell order, so that nothing is merged
+// and a list's particles are read where they lie, not through the order
+// (18M clustered particles at 256^3: 0.84 ms merged,
+// 0.50).  CELL_SHORT 128, 256 and 512 here gave the deposit 0, 1 and 4% more.
+template <bool INORDER>
 __global__ void __launch_bounds__(256)
 k_cic_cells(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *__restrict__ end,
             const int32_t *__restrict__ idx, const float *__restrict__ x,
@@ -486,10 +520,23 @@ k_cic_cells(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *__re
     long_k[slot] = K;
     return;
   }
+  float r = 0.f;
+  if constexpr (INORDER) {
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const int q = kCornerByKey[o];
+      for (int32_t nn = s[q]; nn < e[q]; ++nn) {
+        float ab, de, gh;
+        weights(x[nn], y[nn], z[nn], ab, de, gh);
+        r = cic_add(r, corner_term(q, c, ab, de, gh));
+      }
+    }
+    rho[cid] = r;
+    return;
+  }
   int32_t hv[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) hv[q] = s[q] < e[q] ? idx[s[q]] : INT_MAX;
-  float r = 0.f;
   for (int t = 0; t < K; ++t) {
     const int qs = merge_pick(hv);
     const int32_t nn = hv[qs];
@@ -508,9 +555,16 @@ k_cic_cells(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *__re
 // it -- the merge is the lists in the order of their first particles, and
 // all lanes form the terms; otherwise lane 0 merges them one contribution
 // at a time, its merge state carried across chunks.  A wave per workgroup
-// keeps many cells' latency-bound sums in flight on each CU.
+// keeps many cells' latency-bound sums in flight on each CU.  INORDER: as in
+// k_cic_cells, the lists follow each other in kCornerByKey's order, and each
+// lane forms its own terms, without LDS.  18M clustered particles at 256^3
+// (73,000 long cells, 70M contributions, the longest cell 33,600): 1.91 ms
+// merged with lane 0's setup and the scan by LDS permutes, 1.48 with the
+// lists in order, 0.98 with the scan by lane moves, the first terms added
+// directly and the next particles' loads in flight.
 constexpr int LC_CHUNK = 2 * 64 * LT;
 
+template <bool INORDER>
 __global__ void __launch_bounds__(64)
 k_cic_long_sum(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *__restrict__ end,
                const int32_t *__restrict__ idx, const uint32_t *__restrict__ long_cell,
@@ -526,7 +580,26 @@ k_cic_long_sum(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *_
     const uint32_t cid = long_cell[t];
     const int64_t K = long_k[t];
     int32_t s[8], e[8], hv[8];  // lane 0's merge state
-    if (tid == 0) {
+    if constexpr (INORDER) {
+      if (tid < 8) {
+        const int q = kCornerByKeyDev[tid];
+        const int k = (int)(cid % (uint32_t)g.ng2);
+        const uint32_t ij = cid / (uint32_t)g.ng2;
+        const int j = (int)(ij % (uint32_t)g.ng1), i = (int)(ij / (uint32_t)g.ng1);
+        const uint32_t b = ((uint32_t)(i - kCornerDx[q] + 1) * ex.e1 + (uint32_t)(j - kCornerDy[q] + 1)) * ex.e2 +
+                           (uint32_t)(k - kCornerDz[q] + 1);
+        const int32_t sb = beg[b], len = end[b] - sb;
+        int32_t off = len;
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) {
+          const int32_t o = __shfl_up(off, d);
+          if (tid >= d) off += o;
+        }
+        ss[q] = sb;
+        se[q] = sb + len;
+        soff[q] = off - len;
+      }
+    } else if (tid == 0) {
       const int k = (int)(cid % (uint32_t)g.ng2);
       const uint32_t ij = cid / (uint32_t)g.ng2;
       const int j = (int)(ij % (uint32_t)g.ng1), i = (int)(ij / (uint32_t)g.ng1);
@@ -564,6 +637,48 @@ k_cic_long_sum(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *_
     }
     __syncthreads();
     float r = 0.f;
+    if constexpr (INORDER) {
+      // a lane's terms straight from the lists; the next step's particles
+      // are on their way while this one's terms are added
+      float px[LT], py[LT], pz[LT];
+      int pq[LT];
+      auto fetch = [&](int64_t c0) {
+#pragma unroll
+        for (int k = 0; k < LT; ++k) {
+          const int64_t pos = c0 + LT * tid + k;
+          int q = -1;
+          int32_t nn = 0;
+#pragma unroll
+          for (int qq = 0; qq < 8; ++qq) {
+            const int64_t at = pos - soff[qq];
+            if (at >= 0 && at < se[qq] - ss[qq]) {
+              q = qq;
+              nn = ss[qq] + (int32_t)at;
+            }
+          }
+          pq[k] = q;  // -1 past the last
+          px[k] = x[nn];
+          py[k] = y[nn];
+          pz[k] = z[nn];
+        }
+      };
+      fetch(0);
+      for (int64_t c0 = 0; c0 < K; c0 += 64 * LT) {
+        const int cnt = (int)min<int64_t>(64 * LT, K - c0);
+        double tt[LT];
+#pragma unroll
+        for (int k = 0; k < LT; ++k) {
+          float ab, de, gh;
+          weights(px[k], py[k], pz[k], ab, de, gh);
+          tt[k] = pq[k] >= 0 ? corner_term(pq[k], c, ab, de, gh) : 0.0;
+        }
+        if (c0 + 64 * LT < K) fetch(c0 + 64 * LT);
+        r = c0 == 0 ? wave_add_step<true>(r, tt, cnt) : wave_add_step<false>(r, tt, cnt);
+      }
+      if (tid == 0) rho[cid] = r;
+      __syncthreads();  // the lists are rewritten for the next cell
+      continue;
+    }
     for (int64_t c0 = 0; c0 < K; c0 += LC_CHUNK) {
       const int cl = (int)min<int64_t>(LC_CHUNK, K - c0);
       if (disjoint) {
@@ -603,7 +718,7 @@ k_cic_long_sum(Grid g, Ext ex, const int32_t *__restrict__ beg, const int32_t *_
             const int i = LT * tid + k;
             tt[k] = i < cnt ? tb[b + i] : 0.0;
           }
-          r = wave_add_step(r, tt, cnt);
+          r = c0 + b == 0 ? wave_add_step<true>(r, tt, cnt) : wave_add_step<false>(r, tt, cnt);
         }
       }
       __syncthreads();  // tb is rewritten by the next chunk
@@ -719,7 +834,7 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   // run key; the long-cell counter
   const size_t nn = (size_t)n, nc = (size_t)g.safe, ms = 8 * nn, ne = (size_t)ex.out;
   // (each array starts on a 256-byte boundary: 14 arrays)
-  const size_t bytes = 8 * (nc + ms) + 4 * (6 * nn + 2 * ne + nc + ms) + 8 + 14 * 256;
+  const size_t bytes = 8 * (nc + ms) + 4 * (6 * nn + 2 * ne + nc + ms) + 16 + 14 * 256;
   HSR_HIP(dbuf_reserve(c->sub.keys, bytes));
   char *bp = (char *)c->sub.keys.p;
   auto take = [&bp](size_t b) {
@@ -739,39 +854,54 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   int32_t *end = (int32_t *)take(4 * ne);
   uint32_t *long_cell = (uint32_t *)take(4 * nc);
   uint32_t *skey = (uint32_t *)take(4 * ms);
-  unsigned long long *nlong = (unsigned long long *)take(8);
+  unsigned long long *nlong = (unsigned long long *)take(16);  // and the unsorted flag
+  int32_t *unsorted = (int32_t *)(nlong + 1);
   if ((size_t)(bp - (char *)c->sub.keys.p) > c->sub.keys.bytes) {
     hsr_set_error("hsr_cic: staging layout exceeds its buffer");
     return HSR_ERR_STATE;
   }
   k_zero_u64<<<1, 64, 0, st>>>(nlong);
+  k_zero_u64<<<1, 64, 0, st>>>(nlong + 1);
   // particles by base cell (stable)
-  k_cic_base<<<nblk(n, 256), 256, 0, st>>>(n, x, y, z, g, ex, key, idx, nout);
-  size_t tmp = 0;
-  HSR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key2, idx, idx2, (int)n, 0, bits, st));
-  HSR_HIP(dbuf_reserve(c->s.cub, tmp + 256));
-  HSR_HIP(hipcub::DeviceRadixSort::SortPairs(c->s.cub.p, tmp, key, key2, idx, idx2, (int)n, 0, bits, st));
-  k_fill_i32<<<nblk((int64_t)ne, 256), 256, 0, st>>>((int64_t)ne, beg);
-  k_fill_i32<<<nblk((int64_t)ne, 256), 256, 0, st>>>((int64_t)ne, end);
-  k_cic_ranges<<<nblk(n, 256), 256, 0, st>>>(n, key2, ex, beg, end);
-  // short cells summed, long ones queued and summed a workgroup each (the
-  // grid loops over the device-side count)
-  k_cic_cells<<<nblk((int64_t)nc, 256), 256, 0, st>>>(g, ex, beg, end, idx2, x, y, z, cc, rho, long_cell,
-                                                      long_k, nlong);
-  const unsigned lgrid = (unsigned)std::max(1, c->num_cus) * 32;
-  k_cic_long_sum<<<lgrid, 64, 0, st>>>(g, ex, beg, end, idx2, long_cell, long_k, nlong, x, y, z, cc, rho);
-  // the outside slot: its contributions in (particle, corner) order
+  k_cic_base<<<nblk(n, 256), 256, 0, st>>>(n, x, y, z, g, ex, key, idx, nout, unsorted);
+  // the outside slot's contributions, and whether there is anything to sort:
+  // one host round trip, which the contributions' count takes anyway
   hsr_status s;
   if ((s = pm_excl_scan(c, nout, out_base, n)) != HSR_OK) return s;
-  int32_t last[2] = {0, 0};
+  int32_t last[3] = {0, 0, 0};
   HSR_HIP(hipMemcpyAsync(&last[0], out_base + n - 1, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   HSR_HIP(hipMemcpyAsync(&last[1], nout + n - 1, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  HSR_HIP(hipMemcpyAsync(&last[2], unsorted, sizeof(int32_t), hipMemcpyDeviceToHost, st));
   HSR_HIP(stream_wait(st));
   const int64_t m = (int64_t)last[0] + last[1];
   if ((size_t)m > ms) {
     hsr_set_error("hsr_cic: staged contributions exceed 8 per particle");
     return HSR_ERR_STATE;
   }
+  if (last[2]) {
+    size_t tmp = 0;
+    HSR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key2, idx, idx2, (int)n, 0, bits, st));
+    HSR_HIP(dbuf_reserve(c->s.cub, tmp + 256));
+    HSR_HIP(hipcub::DeviceRadixSort::SortPairs(c->s.cub.p, tmp, key, key2, idx, idx2, (int)n, 0, bits, st));
+  } else {
+    // as the resort leaves them: particles in cell order have their base
+    // cells in order, and a stable sort would move nothing (18M particles at
+    // 256^3: 0.8 ms)
+    key2 = key;
+    idx2 = idx;
+  }
+  k_fill_i32<<<nblk((int64_t)ne, 256), 256, 0, st>>>((int64_t)ne, beg);
+  k_fill_i32<<<nblk((int64_t)ne, 256), 256, 0, st>>>((int64_t)ne, end);
+  k_cic_ranges<<<nblk(n, 256), 256, 0, st>>>(n, key2, ex, beg, end);
+  // short cells summed, long ones queued and summed a workgroup each (the
+  // grid loops over the device-side count)
+  const auto cells = last[2] ? &k_cic_cells<false> : &k_cic_cells<true>;
+  cells<<<nblk((int64_t)nc, 256), 256, 0, st>>>(g, ex, beg, end, idx2, x, y, z, cc, rho, long_cell, long_k,
+                                                nlong);
+  const unsigned lgrid = (unsigned)std::max(1, c->num_cus) * 32;
+  const auto long_sum = last[2] ? &k_cic_long_sum<false> : &k_cic_long_sum<true>;
+  long_sum<<<lgrid, 64, 0, st>>>(g, ex, beg, end, idx2, long_cell, long_k, nlong, x, y, z, cc, rho);
+  // the outside slot: its contributions in (particle, corner) order
   if (m > 0) {
     k_cic_out_terms<<<nblk(n, 256), 256, 0, st>>>(n, x, y, z, g, cc, nout, out_base, 0, skey, ts);
     k_cic_tail<<<1, TAIL_THREADS, 0, st>>>(m, skey, ts, rho);

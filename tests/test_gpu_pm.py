@@ -76,6 +76,34 @@ def test_cic_deposit_orders(order):
     assert bad.size == 0, f"cells differ: {bad[:5]} ({got[bad[:3]]} vs {want[bad[:3]]})"
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 20000])
+@pytest.mark.parametrize("order", ["cells", "swap", "outside inside", "reversed"])
+def test_cic_base_cells_in_order(n, order):
+    """Particles whose base cells come in order need no sort: all in order
+    with the outside ones last, one pair swapped across a wave's edge, one
+    outside particle in the middle, and the whole order reversed, at counts
+    around a wave's and a workgroup's.  Bit-exact."""
+    say(f"case cic base cells n {n} order {order}")
+    ng = (12, 9, 10)
+    x, y, z = positions(n, ng, 31, clump=0.3)
+    ix, iy, iz = (np.floor(a).astype(np.int64) for a in (x, y, z))
+    inb = (ix >= -1) & (ix < ng[0]) & (iy >= -1) & (iy < ng[1]) & (iz >= -1) & (iz < ng[2])
+    key = ((ix + 1) * (ng[1] + 1) + iy + 1) * (ng[2] + 1) + iz + 1
+    perm = np.argsort(np.where(inb, key, 1 << 40), kind="stable")
+    if order == "swap" and n > 64:
+        perm[[63, 64]] = perm[[64, 63]]
+    elif order == "outside inside":
+        perm = np.roll(perm, n // 2)
+    elif order == "reversed":
+        perm = perm[::-1]
+    x, y, z = x[perm].copy(), y[perm].copy(), z[perm].copy()
+    want = O.cic(x, y, z, ng, gpscal=0.75)
+    ctx = Context()
+    got = ctx.cic(x, y, z, ng, gpscal=0.75)
+    ctx.close()
+    assert (bits(got) == bits(want)).all()
+
+
 def test_cic_device_tensors_and_reuse():
     """Device arrays in place; a second call on the same grid starts from
     zero again."""
