@@ -104,6 +104,29 @@ def test_cic_base_cells_in_order(n, order):
     assert (bits(got) == bits(want)).all()
 
 
+@pytest.mark.parametrize("length", [9, 63, 64, 65, 128, 129, 1000])
+@pytest.mark.parametrize("skew", [0, 1])
+def test_cic_interleaved_lists(length, skew):
+    """A long cell whose eight lists interleave, lists around the merge's
+    window of 64, equal or (skew) one of them many times the others', and
+    among them empty ones.  Bit-exact."""
+    say(f"case cic interleaved lists of {length} skew {skew}")
+    rng = np.random.default_rng(41)
+    ng = (5, 5, 5)
+    base = np.stack(np.meshgrid([1, 2], [1, 2], [1, 2], indexing="ij"), -1).reshape(8, 3)
+    cnt = np.full(8, length)
+    if skew:
+        cnt = np.array([10 * length, 0, length, 1, length + 1, 0, 2, length])
+    p = np.concatenate([b + rng.uniform(0, 1, (c, 3)) for b, c in zip(base, cnt)])
+    p = np.minimum(p, 2.999).astype(np.float32)[rng.permutation(p.shape[0])]
+    x, y, z = (p[:, k].copy() for k in range(3))
+    want = O.cic(x, y, z, ng, gpscal=1.0)
+    ctx = Context()
+    got = ctx.cic(x, y, z, ng, gpscal=1.0)
+    ctx.close()
+    assert (bits(got) == bits(want)).all()
+
+
 def test_cic_device_tensors_and_reuse():
     """Device arrays in place; a second call on the same grid starts from
     zero again."""
