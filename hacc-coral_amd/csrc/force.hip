@@ -711,8 +711,7 @@ LawArgs law_args(const ForceLawDev &D) {
 }  // namespace
 
 // Target order inside each listed leaf: positions sorted along the leaf's
-// longest box edge (ties x > y > z; coordinates equal in their leading
-// 22 bits by position), so that
+// longest box edge (ties x > y > z; equal coordinates by position), so that
 // a pass's 128 targets span a slab of the leaf and the entries its box is
 // beyond the cutoff of can be skipped.  iperm[off + k] = position of the
 // k-th target; leaves above SORT_MAX keep their order.
@@ -725,9 +724,10 @@ __global__ void k_iota32(int64_t n, int32_t *a) {
 
 // Every target's place is the number of smaller keys in its leaf: n broadcast
 // LDS reads a target and no barriers, where a bitonic sort took log^2 n of
-// them (0.68 -> 0.41 ms at 256^3 with leaves of 512).  The keys are the
-// coordinate's leading 22 bits, then the position, so no two are equal; the
-// passes need no finer order.
+// them (0.68 -> 0.41 ms at 256^3 with leaves of 512).  The keys
+// are whole coordinates: with their leading 22 bits alone dense leaves come
+// out unordered, their passes' boxes grow, and the fused adjoint took 474 ms
+// instead of 455 at 256^3.
 __global__ void __launch_bounds__(256)
 k_leaf_sort(int64_t nl, const int32_t *__restrict__ leaves, const hsr_node *__restrict__ cn,
             const PJ *__restrict__ pj, int32_t *__restrict__ iperm) {
@@ -745,15 +745,20 @@ k_leaf_sort(int64_t nl, const int32_t *__restrict__ leaves, const hsr_node *__re
     const PJ p = pj[off + i];
     const uint32_t u = __float_as_uint(d == 0 ? p.x : (d == 1 ? p.y : p.z));
     // an unsigned number in the order of the floats
-    const uint32_t ord = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
-    key[i] = (ord & ~(uint32_t)(SORT_MAX - 1)) | (uint32_t)i;
+    key[i] = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
   }
   __syncthreads();
   for (int i = threadIdx.x; i < cnt; i += 256) {
     const uint32_t mine = key[i];
+    // equal coordinates by position: those before count, those after do not
+    const int w0 = i & ~63, w1 = min(w0 + 64, cnt);  // the wave's own
     int rank = 0;
 #pragma unroll 8
-    for (int q = 0; q < cnt; ++q) rank += key[q] < mine ? 1 : 0;
+    for (int q = 0; q < w0; ++q) rank += key[q] <= mine ? 1 : 0;
+#pragma unroll 8
+    for (int q = w0; q < w1; ++q) rank += key[q] < mine || (key[q] == mine && q < i) ? 1 : 0;
+#pragma unroll 8
+    for (int q = w1; q < cnt; ++q) rank += key[q] < mine ? 1 : 0;
     iperm[off + rank] = (int32_t)(off + i);
   }
 }
