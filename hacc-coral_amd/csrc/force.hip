@@ -412,7 +412,10 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
 }
 
 // Sum the chunk partials of long lists in chunk order; the last workgroup
-// sums the waves' pair counts (the waves past the items counted none).
+// sums the waves' pair counts: of every wave, since one past the items' number
+// pops items too while the queue's owners (half the waves) are fewer than the
+// items; with no more items than owners nothing is popped and the waves past
+// the items counted none.
 __global__ void __launch_bounds__(256)
 k_reduce_chunks(const hsr_node *cn, const int32_t *leaves,
                 const int64_t *multi, const int64_t *nmulti_p,
@@ -422,7 +425,7 @@ k_reduce_chunks(const hsr_node *cn, const int32_t *leaves,
                 unsigned long long *totals) {
   if (blockIdx.x == gridDim.x - 1) {
     if (threadIdx.x >= 64) return;
-    const int64_t nw = min(nwaves, *nitems_p);
+    const int64_t nw = *nitems_p <= nwaves / 2 ? *nitems_p : nwaves;
     uint64_t a = 0, b = 0;
 #pragma unroll 8
     for (int64_t w = threadIdx.x; w < nw; w += 64) {
