@@ -2034,21 +2034,71 @@ __device__ __forceinline__ float pp12_term(float x, float y, float z, float w,
   return w * (odr0 + odr1 + odr2);
 }
 
+// Node ids by depth, for trees whose ids are not in level order (subtrees):
+// counts, their prefix (start[d], one more entry than depths), places.  The
+// lanes of a wave that share a depth take one atomic.
+__global__ void k_depth_count(const BNode *nodes, int64_t nb, int32_t *count) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int d = t < nb ? nodes[t].depth : -1;
+  uint64_t left = __ballot(d >= 0);
+  while (left) {
+    const int dl = __builtin_amdgcn_readlane(d, (int)__builtin_ctzll(left));
+    const uint64_t same = __ballot(d == dl);
+    if (lane_id() == 0) atomicAdd(&count[dl], (int32_t)__popcll(same));
+    left &= ~same;
+  }
+}
+
+__global__ void __launch_bounds__(64) k_depth_scan(int ndepth, const int32_t *count, int32_t *start,
+                                                   int32_t *next) {
+  const int l = lane_id();
+  int32_t base = 0;
+  for (int d0 = 0; d0 < ndepth; d0 += 64) {
+    const int32_t c = d0 + l < ndepth ? count[d0 + l] : 0;
+    int32_t inc = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t y = __shfl_up(inc, o);
+      if (l >= o) inc += y;
+    }
+    if (d0 + l < ndepth) start[d0 + l] = next[d0 + l] = base + inc - c;
+    base += __builtin_amdgcn_readlane(inc, 63);
+  }
+  if (l == 0) start[ndepth] = base;
+}
+
+__global__ void k_depth_place(const BNode *nodes, int64_t nb, int32_t *next, int32_t *order) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int d = t < nb ? nodes[t].depth : -1;
+  uint64_t left = __ballot(d >= 0);
+  while (left) {
+    const int dl = __builtin_amdgcn_readlane(d, (int)__builtin_ctzll(left));
+    const uint64_t same = __ballot(d == dl);
+    int32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(&next[dl], (int32_t)__popcll(same));
+    base = readlane_i32(base, 0);
+    if (d == dl) order[base + __popcll(same & lanemask_lt())] = (int32_t)t;
+    left &= ~same;
+  }
+}
+
+__global__ void k_zero_i32(int64_t n, int32_t *a) {
+  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (k < n) a[k] = 0;
+}
+
 // pp<12> of every node of one depth (deepest first), one thread
-// per (node, design point): leaves with count > 12 from their members
+// per (node, design point) -- the nodes [lo, hi), of them with depth >= 0 those
+// of that depth, or with `order` the nodes at start[0] .. start[1] of it (the
+// grid strides over them: their number is on the device): leaves with count > 12 from their members
 // (RCBForceTree.cxx:787-797), split nodes from each child, left then right
 // -- its members when count <= 12, else its 12 pseudo-particles
 // (:856-889) -- accumulated in that order; degenerate nodes and leaves with
 // count <= 12 keep 0.  Reads the canonical nodes and the particles in tree
 // order; writes ppm12[12 * canonical id + j].
-__global__ void k_pp12_level(const BNode *nodes, int64_t nb, int depth,
-                             const int64_t *box_cbase, const int32_t *box_of,
-                             hsr_node *cn, const float *xs, const float *ys,
-                             const float *zs, const float *ms, float *ppm12) {
-  const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t t = g / 12;
-  const int j = (int)(g % 12);
-  if (t >= nb || nodes[t].depth != depth) return;
+__device__ __forceinline__ void pp12_node(const BNode *nodes, int64_t t, int j, const int64_t *box_cbase, 
+                                          const int32_t *box_of, hsr_node *cn, const float *xs,
+                                          const float *ys, const float *zs, const float *ms,
+                                          float *ppm12) {
   const BNode &b = nodes[t];
   const int64_t k = box_cbase[box_of[t]] + b.canon;
   const hsr_node &o = cn[k];
@@ -2081,6 +2131,22 @@ __global__ void k_pp12_level(const BNode *nodes, int64_t nb, int depth,
   }
   ppm12[12 * k + j] = acc;
   if (j == 0) cn[k].ppm[0] = acc;  // the node table's mass slot holds ppm[0] of the 12
+}
+
+__global__ void k_pp12_level(const BNode *nodes, int64_t lo, int64_t hi, int depth,
+                             const int32_t *order, const int32_t *start, const int64_t *box_cbase, const int32_t *box_of,
+                             hsr_node *cn, const float *xs, const float *ys, const float *zs,
+                             const float *ms, float *ppm12) {
+  if (order) {
+    lo = start[0];
+    hi = start[1];
+  }
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t g = 12 * lo + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < 12 * hi; g += stride) {
+    const int64_t t = g / 12;
+    if (depth >= 0 && nodes[t].depth != depth) continue;
+    pp12_node(nodes, order ? order[t] : t, (int)(g % 12), box_cbase, box_of, cn, xs, ys, zs, ms, ppm12);
+  }
 }
 
 // Pseudo-particle records of TDPTS = 12: node k's design point j at
@@ -2523,11 +2589,33 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
     HSR_HIP(dbuf_reserve(T.ppm12, sizeof(float) * 12 * std::max<int64_t>(T.nnodes, 1)));
     float *ppm12 = dptr<float>(T.ppm12);
     if (T.nnodes > 0) k_zero_f32<<<nblk_for(12 * T.nnodes, 256), 256, 0, st>>>(12 * T.nnodes, ppm12);
-    for (int64_t d = T.max_depth; d >= 0; --d) {
-      if (nb > 0)
-        k_pp12_level<<<nblk_for(12 * nb, 256), 256, 0, st>>>(
-            nodes, nb, (int)d, d_cbase, box_of, cn, dptr<float>(T.xs), dptr<float>(T.ys), dptr<float>(T.zs),
-            dptr<float>(T.ms), ppm12);
+    const int ndepth = (int)T.max_depth + 1;
+    // Without subtrees a depth is a range of ids.  With them its nodes are
+    // bucketed first (four launches, 15 us) or picked out of all nodes at
+    // every depth (0.02 ns per node and depth: 5.5 ms where a visit of every
+    // node takes 1.2, for 3M nodes of 76 depths; 2.4 us by that rate for 8000
+    // nodes of 16 depths), whichever is less.
+    int32_t *order = nullptr, *start = nullptr;
+    if (nb > upper && nb * ndepth > (int64_t)1 << 20) {
+      HSR_HIP(dbuf_reserve(S.g, sizeof(int32_t) * (size_t)(nb + 3 * ((int64_t)ndepth + 1))));
+      order = dptr<int32_t>(S.g);
+      start = order + nb;
+      int32_t *count = start + ndepth + 1, *next = count + ndepth + 1;
+      k_zero_i32<<<nblk_for(ndepth, 256), 256, 0, st>>>(ndepth, count);
+      k_depth_count<<<nblk_for(nb, 256), 256, 0, st>>>(nodes, nb, count);
+      k_depth_scan<<<1, 64, 0, st>>>(ndepth, count, start, next);
+      k_depth_place<<<nblk_for(nb, 256), 256, 0, st>>>(nodes, nb, next, order);
+    }
+    for (int d = ndepth - 1; d >= 0; --d) {
+      const bool all = nb > upper;
+      const int64_t lo = all ? 0 : T.level_start[d], hi = all ? nb : T.level_start[d + 1];
+      if (hi <= lo) continue;
+      unsigned grid = nblk_for(12 * (hi - lo), 256);
+      if (order) grid = std::min(grid, (unsigned)std::max(1, c->num_cus) * 8);
+      k_pp12_level<<<grid, 256, 0, st>>>(nodes, lo, hi, all && !order ? d : -1, order,
+                                         order ? start + d : nullptr, d_cbase, box_of, cn,
+                                         dptr<float>(T.xs), dptr<float>(T.ys), dptr<float>(T.zs),
+                                         dptr<float>(T.ms), ppm12);
     }
     if (T.nnodes > 0)
       k_pseudo_pj12<<<nblk_for(12 * T.nnodes, 256), 256, 0, st>>>(n, T.nnodes, cn, ppm12, dptr<PJ>(T.pj));
