@@ -1509,20 +1509,19 @@ __global__ void k_box_of(const BNode *nodes, int64_t nb, int32_t *box_of) {
 // read, so a launch that runs out of node slots is repeated with more.
 //
 // A workgroup takes 12 to 15 us a level (dependent integer chains and
-// barriers; 97 KB of LDS, one workgroup a compute unit), so it pays where
+// barriers; 111 KB of LDS, one workgroup a compute unit), so it pays where
 // the levels it replaces are bound by their launches: builds of up to SUB_N
 // particles.  Build time without and with it: 0.99 and 0.63 ms for 12k
 // particles (leaves of 32), 1.93 and 1.62 ms for 365k (leaves of 128), but
 // 3.95 and 4.10 ms for 2.5M (leaves of 256), 9.78 and 10.58 ms for 18M.
 constexpr int SUB_T = 1024;
 constexpr int64_t SUB_N = (int64_t)1 << 20;
-constexpr int SUB_LEVELS = 48;  // levels of a subtree (a deeper one sends the build
-                                // to the level passes)
+constexpr int SUB_LEVELS = SUB_MAX;  // every level but a subtree's first follows a
+                                     // split, which takes a particle off its node
 
 struct SubCtr {
   int64_t next;      // next free node slot
   int32_t overflow;  // a workgroup found no slots
-  int32_t deep;      // a subtree has more than SUB_LEVELS levels
   int64_t depth;     // deepest level used
 };
 
@@ -1545,7 +1544,7 @@ __global__ void k_sub_gather(const BNode *nodes, int64_t nb, int2 *list, int32_t
 __global__ void k_sub_init(SubCtr *c, int64_t next, int32_t *count) {
   if (threadIdx.x == 0) {
     c->next = next;
-    c->overflow = c->deep = 0;
+    c->overflow = 0;
     c->depth = 0;
     if (count) *count = 0;
   }
@@ -1581,8 +1580,8 @@ k_subtree(BNode *nodes, const int2 *__restrict__ list, SubArrays A, int64_t nd, 
   __shared__ float npiv[SUB_MAX];
   __shared__ uint64_t mask[WORDS], smask[WORDS];   // key < pivot; node splits
   __shared__ int32_t wpre[WORDS + 1], spre[WORDS + 1];
-  __shared__ int64_t lbase[SUB_LEVELS];
-  __shared__ int32_t lcnt[SUB_LEVELS], lfirst[SUB_LEVELS];
+  __shared__ int32_t lbase[SUB_LEVELS];            // ids are 32-bit (BNode.cl)
+  __shared__ uint16_t lcnt[SUB_LEVELS], lfirst[SUB_LEVELS];
   __shared__ int64_t base_sh;
   __shared__ int32_t stop_sh;
   const int t = threadIdx.x, w = t >> 6, l = lane_id();
@@ -1613,14 +1612,10 @@ k_subtree(BNode *nodes, const int2 *__restrict__ list, SubArrays A, int64_t nd, 
   int64_t base = root;
   int nn = 1, cur = 0, lev = 0, first = 0;
   while (nn > 0) {
-    if (lev == SUB_LEVELS) {
-      if (t == 0) ctr->deep = 1;
-      return;
-    }
     if (t == 0) {
-      lbase[lev] = base;
-      lcnt[lev] = nn;
-      lfirst[lev] = first;
+      lbase[lev] = (int32_t)base;
+      lcnt[lev] = (uint16_t)nn;
+      lfirst[lev] = (uint16_t)first;
     }
     // ---- bbox, exact sums, centre of mass, class: a wave per node, at the
     // top levels after a wave per SUB_CH elements of it
@@ -2244,12 +2239,9 @@ inline unsigned nblk_for(int64_t n, int t) {
 
 }  // namespace
 
-// The last levels by k_subtree where it can (subtrees), else by the level
-// passes alone.
-static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_off_h,
-                               const float *min_loc_h, const float *max_loc_h, const float *x,
-                               const float *y, const float *z, const float *m, bool subtrees,
-                               bool *too_deep) {
+hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes, const int64_t *box_off_h,
+                             const float *min_loc_h, const float *max_loc_h, const float *x,
+                             const float *y, const float *z, const float *m) {
   hipStream_t st = c->stream;
   TreeState &T = c->tree;
   Scratch &S = c->s;
@@ -2324,7 +2316,7 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
   int64_t active = n;
   Counters hc;
   int depth = 0;
-  const bool use_sub = subtrees && unit && n <= SUB_N;
+  const bool use_sub = unit && n <= SUB_N;
   // whether the level holds nodes above CM_SMALL, up to it, and leaves for the
   // level passes to finish (with subtrees, k_subtree takes all up to SUB_MAX)
   bool run_big = false, run_small = !use_sub, run_leaf = true;
@@ -2503,10 +2495,6 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
       SubCtr hs;
       HSR_HIP(hipMemcpyAsync(&hs, sub_ctr, sizeof(SubCtr), hipMemcpyDeviceToHost, st));
       HSR_HIP(stream_wait(st));
-      if (hs.deep) {
-        *too_deep = true;
-        return HSR_OK;
-      }
       if (!hs.overflow) {
         T.nnodes_bfs = hs.next;
         T.max_depth = std::max(T.max_depth, hs.depth);
@@ -2624,14 +2612,4 @@ static hsr_status build_levels(hsr_ctx *c, int64_t nboxes, const int64_t *box_of
   }
   HSR_HIP(hipGetLastError());
   return HSR_OK;
-}
-
-hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes, const int64_t *box_off, const float *min_loc,
-                             const float *max_loc, const float *x, const float *y, const float *z,
-                             const float *m) {
-  bool too_deep = false;
-  hsr_status s = build_levels(c, nboxes, box_off, min_loc, max_loc, x, y, z, m, true, &too_deep);
-  if (s == HSR_OK && too_deep)
-    s = build_levels(c, nboxes, box_off, min_loc, max_loc, x, y, z, m, false, &too_deep);
-  return s;
 }

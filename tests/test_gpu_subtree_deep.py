@@ -1,0 +1,52 @@
+"""Subtrees of one workgroup that are deep: bit-exact with the oracle, and
+built by the workgroup, not by the passes over levels."""
+import numpy as np
+import pytest
+
+from haccsr import Context
+from test_gpu_subtree import oracle_tree, same
+
+pytestmark = pytest.mark.gpu
+
+
+def chain(per_axis, ratio, n):
+    """per_axis particles in geometric sequence on each axis, n more spread."""
+    rng = np.random.default_rng(per_axis)
+    k = np.arange(3 * per_axis)
+    geo = np.stack([np.where(k % 3 == d, ratio ** (k // 3), 0.0) for d in range(3)], 1)
+    return np.concatenate([geo, 1.0 + 7.0 * rng.random((n, 3))]).astype(np.float32)
+
+
+@pytest.mark.parametrize("per_axis,ratio,n,nd", [(40, 0.4, 0, 1), (95, 0.3, 0, 1), (95, 0.3, 40000, 3),
+                                                 (650, 0.9, 0, 1)])
+def test_deep(per_axis, ratio, n, nd):
+    p = chain(per_axis, ratio, n)
+    ref = oracle_tree(p, 8.0, nd)
+    ctx = Context(nd=nd)
+    x, y, z = (p[:, k].copy() for k in range(3))
+    ids = np.arange(p.shape[0], dtype=np.int64)
+    ctx.build(x, y, z, np.ones(p.shape[0], np.float32), ids=ids, min_loc=(0, 0, 0), max_loc=(8, 8, 8))
+    print(f"case subtree deep n={p.shape[0]} depth {ctx.stats().max_depth}", flush=True)
+    assert np.array_equal(ids, ref.id)
+    same(ctx.nodes(), ref.nodes)
+    for f in ("offset", "cl", "cr"):
+        assert np.array_equal(ctx.nodes()[f], ref.nodes[f]), f
+    ctx.close()
+
+
+def test_deep_tree_is_built_once():
+    p = chain(95, 0.3, 0)
+    ms = []
+    for mass in (1.0, 0.5):  # one subtree; the passes over levels
+        ctx = Context(nd=1)
+        best = np.inf
+        for _ in range(4):
+            x, y, z = (p[:, k].copy() for k in range(3))
+            ctx.build(x, y, z, np.full(p.shape[0], mass, np.float32), min_loc=(0, 0, 0), max_loc=(8, 8, 8))
+            best = min(best, ctx.stats().build_ms)
+        ms.append(best)
+        print(f"case subtree deep mass {mass} depth {ctx.stats().max_depth} build {best:.3f} ms", flush=True)
+        assert ctx.stats().max_depth > 60
+        ctx.close()
+    # a level: 12 to 15 us by a workgroup, more than 50 us by the passes
+    assert ms[0] < 0.75 * ms[1]
