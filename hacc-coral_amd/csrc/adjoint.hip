@@ -1036,6 +1036,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
     const size_t wbytes = sizeof(float) * 3 * (size_t)(LS.nentries + 1);
     size_t free_b = 0, total_b = 0;
     HSR_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += dbuf_kept_bytes();  // given back to an allocation that needs them
     const bool fits = wbytes <= A.W.bytes || (double)wbytes <= 0.7 * (double)free_b;
     const int mode = c->tuning.adjoint_mode;
     A.fused = mode == 1 || (mode == 0 && fits);

@@ -355,9 +355,11 @@ namespace {
 // back and half as much to get (a 48^3 step through the constructor: 6.2 ms,
 // 4.1 with the buffers kept).
 // Bounded: at most KEEP_BYTES a device, none above KEEP_ONE, the oldest
-// freed first; all are given back when an allocation fails.  A buffer enters
-// only after its context's stream has been waited for (hsr_destroy), so the
-// next owner may use it on any stream.
+// freed first; all are given back when an allocation of this library fails,
+// and to the rest of the process by hsr_release_buffers.  A buffer enters
+// only after its context's stream has been waited for without an error
+// (hsr_destroy), so the next owner may use it on any stream.  The mutex covers
+// the table alone: buffers are freed (which waits for the device) outside it.
 constexpr size_t KEEP_BYTES = (size_t)1 << 30, KEEP_ONE = (size_t)1 << 28;
 struct Kept {
   void *p;
@@ -392,40 +394,59 @@ void kept_put(void *p, size_t bytes) {
     (void)hipFree(p);
     return;
   }
-  std::lock_guard<std::mutex> lock(g_kept_mutex);
-  g_kept.push_back({p, bytes, dev});
-  size_t total = 0;
-  for (const Kept &k : g_kept) total += k.device == dev ? k.bytes : 0;
-  for (size_t i = 0; total > KEEP_BYTES && i < g_kept.size();) {
-    if (g_kept[i].device != dev) {
-      ++i;
-      continue;
+  std::vector<void *> out;
+  {
+    std::lock_guard<std::mutex> lock(g_kept_mutex);
+    g_kept.push_back({p, bytes, dev});
+    size_t total = 0;
+    for (const Kept &k : g_kept) total += k.device == dev ? k.bytes : 0;
+    for (size_t i = 0; total > KEEP_BYTES && i < g_kept.size();) {
+      if (g_kept[i].device != dev) {
+        ++i;
+        continue;
+      }
+      total -= g_kept[i].bytes;
+      out.push_back(g_kept[i].p);
+      g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
     }
-    total -= g_kept[i].bytes;
-    (void)hipFree(g_kept[i].p);
-    g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
   }
+  for (void *q : out) (void)hipFree(q);
 }
 
-// Gives every kept buffer of the current device back; whether there was one.
-bool kept_release() {
+// Gives every kept buffer of the current device back; the bytes they held.
+size_t kept_release() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  std::lock_guard<std::mutex> lock(g_kept_mutex);
-  bool any = false;
-  for (size_t i = 0; i < g_kept.size();) {
-    if (g_kept[i].device != dev) {
-      ++i;
-      continue;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::vector<Kept> out;
+  {
+    std::lock_guard<std::mutex> lock(g_kept_mutex);
+    for (size_t i = 0; i < g_kept.size();) {
+      if (g_kept[i].device != dev) {
+        ++i;
+        continue;
+      }
+      out.push_back(g_kept[i]);
+      g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
     }
-    (void)hipFree(g_kept[i].p);
-    g_kept.erase(g_kept.begin() + (ptrdiff_t)i);
-    any = true;
   }
-  return any;
+  size_t bytes = 0;
+  for (const Kept &k : out) {
+    bytes += k.bytes;
+    (void)hipFree(k.p);
+  }
+  return bytes;
 }
 
 }  // namespace
+
+size_t dbuf_kept_bytes() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> lock(g_kept_mutex);
+  size_t total = 0;
+  for (const Kept &k : g_kept) total += k.device == dev ? k.bytes : 0;
+  return total;
+}
 
 hipError_t dbuf_reserve(DBuf &b, size_t bytes) {
   if (bytes <= b.bytes && b.p) return hipSuccess;
@@ -451,7 +472,7 @@ hipError_t dbuf_reserve(DBuf &b, size_t bytes) {
     want = std::max<size_t>(bytes, 256);
     e = hipMalloc(&b.p, want);
   }
-  if (e != hipSuccess && kept_release()) {  // no room beside the kept buffers
+  if (e != hipSuccess && kept_release() > 0) {  // no room beside the kept buffers
     (void)hipGetLastError();
     e = hipMalloc(&b.p, want);
   }
@@ -575,7 +596,7 @@ hsr_status hsr_set_law_table(hsr_ctx *c, const float *r2, const float *f, int64_
 hsr_status hsr_destroy(hsr_ctx *c) {
   if (!c) return HSR_OK;
   (void)hipSetDevice(c->device);
-  (void)hipStreamSynchronize(c->stream);
+  const bool idle = hipStreamSynchronize(c->stream) == hipSuccess;
   DBuf *bufs[] = {&c->tree.bnodes, &c->tree.canon_nodes, &c->tree.pfin, &c->tree.pj, &c->tree.ppm12,
                   &c->tree.xs, &c->tree.ys, &c->tree.zs, &c->tree.ms,
                   &c->lists.leaves, &c->lists.seg_ptr, &c->lists.seg, &c->lists.ent_ptr,
@@ -591,7 +612,8 @@ hsr_status hsr_destroy(hsr_ctx *c) {
                   &c->s.pblocks, &c->s.cnode, &c->s.pnode, &c->s.pmask, &c->s.counters, &c->dev_v, &c->force};
   if (c->adj.graph_exec) (void)hipGraphExecDestroy(c->adj.graph_exec);
   if (c->adj.graph) (void)hipGraphDestroy(c->adj.graph);
-  auto give = [](DBuf &b) {  // idle: the stream has been waited for
+  auto give = [idle](DBuf &b) {
+    if (!idle) return dbuf_free(b);
     if (b.p) kept_put(b.p, b.bytes);
     b.p = nullptr;
     b.bytes = 0;
@@ -611,6 +633,25 @@ hsr_status hsr_destroy(hsr_ctx *c) {
   if (c->graph) (void)hipGraphDestroy(c->graph);
   (void)hipStreamDestroy(c->stream);
   delete c;
+  return HSR_OK;
+}
+
+hsr_status hsr_release_buffers(int device, int64_t *bytes) {
+  if (bytes) *bytes = 0;
+  int ndev = 0, cur = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) {
+    g_err = "hsr_release_buffers: no HIP device available";
+    return HSR_ERR_HIP;
+  }
+  if (device < 0 || device >= ndev) {
+    g_err = "hsr_release_buffers: device ordinal out of range";
+    return HSR_ERR_ARG;
+  }
+  HSR_HIP(hipGetDevice(&cur));
+  HSR_HIP(hipSetDevice(device));
+  const size_t freed = kept_release();
+  HSR_HIP(hipSetDevice(cur));
+  if (bytes) *bytes = (int64_t)freed;
   return HSR_OK;
 }
 

@@ -73,6 +73,8 @@ struct DBuf {
 };
 
 hipError_t dbuf_reserve(DBuf &b, size_t bytes);
+// bytes of the current device that destroyed contexts left for the next ones
+size_t dbuf_kept_bytes();
 void dbuf_free(DBuf &b);
 
 template <class T>

@@ -9,14 +9,14 @@ mirrors the sub-cycle and PM particle-grid methods of the reference's
 Particles class, and ``restart`` reads and writes its restart files.
 """
 from ._lib import (Context, HsrError, LAW_NEWTON, LAW_SR_FIT, LAW_SR_INTERP,
-                   LAW_SR_POLY5, LAW_SR_POLY6, LAW_STEP16, NODE_DTYPE, load)
+                   LAW_SR_POLY5, LAW_SR_POLY6, LAW_STEP16, NODE_DTYPE, load, release_buffers)
 from .forcetree import (FGrid, FGridEvalFit, FGridEvalInterp, FGridEvalPoly,
                         ForceLaw, ForceLawNewton, ForceLawSR, RCBMonopoleForceTree,
                         RCBQuadrupoleForceTree)
 
 __all__ = [
     "Context", "HsrError", "LAW_NEWTON", "LAW_SR_FIT", "LAW_SR_INTERP",
-    "LAW_SR_POLY5", "LAW_SR_POLY6", "LAW_STEP16", "NODE_DTYPE", "load", "FGrid",
-    "FGridEvalFit", "FGridEvalInterp", "FGridEvalPoly", "ForceLaw", "ForceLawNewton", "ForceLawSR",
+    "LAW_SR_POLY5", "LAW_SR_POLY6", "LAW_STEP16", "NODE_DTYPE", "load", "release_buffers",
+    "FGrid", "FGridEvalFit", "FGridEvalInterp", "FGridEvalPoly", "ForceLaw", "ForceLawNewton", "ForceLawSR",
     "RCBMonopoleForceTree", "RCBQuadrupoleForceTree",
 ]

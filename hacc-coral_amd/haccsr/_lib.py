@@ -27,7 +27,7 @@ HSR_OK, HSR_ERR_ARG, HSR_ERR_HIP, HSR_ERR_UNSUPPORTED = 0, 1, 2, 3
 HSR_ERR_STATE, HSR_ERR_NOMEM, HSR_ERR_NUMERIC = 4, 5, 6
 
 EXPORTS = [
-    "hsr_last_error", "hsr_version", "hsr_create", "hsr_destroy",
+    "hsr_last_error", "hsr_version", "hsr_create", "hsr_release_buffers", "hsr_destroy",
     "hsr_get_stream", "hsr_build", "hsr_lists", "hsr_forces", "hsr_kick",
     "hsr_adjoint", "hsr_get_stats", "hsr_get_nodes", "hsr_get_perm",
     "hsr_get_lists", "hsr_build_many", "hsr_lists_many", "hsr_set_tuning",
@@ -143,6 +143,7 @@ def load(path: str | None = None):
     L.hsr_version.restype = C.c_char_p
     L.hsr_create.argtypes = [C.POINTER(C.c_void_p), C.POINTER(Params)]
     L.hsr_destroy.argtypes = [vp]
+    L.hsr_release_buffers.argtypes = [C.c_int, C.POINTER(C.c_int64)]
     L.hsr_get_stream.argtypes = [vp, C.POINTER(C.c_void_p)]
     L.hsr_build.argtypes = [vp, i64] + [vp] * 10 + [vp, vp, C.c_int]
     L.hsr_build_many.argtypes = [vp, i64, vp] + [vp] * 10 + [vp, vp, C.c_int]
@@ -508,6 +509,14 @@ class Context:
         for k, v in kw.items():
             setattr(t, k, int(v))
         check(self.L.hsr_set_tuning(self.h, C.byref(t)), "hsr_set_tuning")
+
+
+def release_buffers(device: int = 0) -> int:
+    """hsr_release_buffers: frees the device buffers that destroyed contexts
+    left for the next ones (at most 1 GiB a device); their bytes."""
+    n = C.c_int64()
+    check(load().hsr_release_buffers(int(device), C.byref(n)), "hsr_release_buffers")
+    return n.value
 
 
 def domain(rL, oL, ng) -> Domain:

@@ -108,6 +108,15 @@ const char *hsr_version(void);
 hsr_status hsr_create(hsr_ctx **ctx, const hsr_params *p);
 hsr_status hsr_destroy(hsr_ctx *ctx);
 
+/* The device buffers of destroyed contexts are kept for the next ones, so a
+ * context a step pays no allocations: at most 1 GiB a device, none above
+ * 256 MiB, the oldest freed first, all of them when an allocation of this
+ * library fails.  Other users of the device (another allocator in the
+ * process, another process) get that memory through this call, which frees
+ * every kept buffer of the device; *bytes (may be NULL) receives their size.
+ * Buffers of live contexts are not touched; from any thread. */
+hsr_status hsr_release_buffers(int device, int64_t *bytes);
+
 /* The table of an HSR_LAW_SR_INTERP context: FGridEvalInterp's r2() and f()
  * arrays of nInterp entries (ForceLaw.h:73-91, filled by
  * FGrid::fgor_r2_interp, ForceLaw.cxx:54-67), copied to the device; n must
