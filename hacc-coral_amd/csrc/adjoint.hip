@@ -977,14 +977,19 @@ T tail_sum(hsr_ctx *c, const T *excl, const T *cnt, int64_t n) {
 
 }  // namespace
 
-// Transposed lists and item queues (once per list build).
-hsr_status adjoint_plan(hsr_ctx *c) {
+// Transposed lists and item queues (once per list build), the lists cut into
+// items of `chunk` entries (full: an allocation found no room).
+static hsr_status adjoint_plan_chunk(hsr_ctx *c, int64_t chunk, bool *full) {
   hipStream_t st = c->stream;
+  auto reserve = [full](DBuf &b, size_t bytes) {
+    const hipError_t e = dbuf_reserve(b, bytes);
+    *full = e == hipErrorOutOfMemory;
+    return e;
+  };
   AdjState &A = c->adj;
   ListState &LS = c->lists;
   TreeState &T = c->tree;
   const int64_t nl = LS.nleaves, ns = LS.nsegs, nn = T.nnodes, n = T.n;
-  const int64_t chunk = LS.chunk > 0 ? LS.chunk : 16384;
   // host sources of asynchronous copies stay alive until the final sync
   int64_t tail_items[4] = {0, 0, 0, 0};
   const hsr_node *cn = dptr<hsr_node>(T.canon_nodes);
@@ -994,7 +999,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   const int64_t *sb = sa + ns + 1;
   hsr_status s;
   // ---- target-pass items (forward entries)
-  HSR_HIP(dbuf_reserve(A.fw, sizeof(int64_t) * 5 * (nl + 2)));
+  HSR_HIP(reserve(A.fw, sizeof(int64_t) * 5 * (nl + 2)));
   int64_t *fnc = dptr<int64_t>(A.fw), *fib = fnc + (nl + 2), *fps = fib + (nl + 2);
   int64_t *fpb = fps + (nl + 2), *ffirst = fpb + (nl + 2);
   k_fw_counts<<<nblk(nl, 256), 256, 0, st>>>(nl, dptr<int64_t>(LS.ent_ptr), leaves, cn, chunk, fnc, fps);
@@ -1004,13 +1009,13 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   const int64_t nfp = tail_sum(c, fpb, fps, nl);
   A.n_fw_items = nfi;
   A.n_fw_leaves = nl;
-  HSR_HIP(dbuf_reserve(A.fw_items, sizeof(AItem) * (nfi + 1)));
+  HSR_HIP(reserve(A.fw_items, sizeof(AItem) * (nfi + 1)));
   k_fw_items<<<nblk(nl, 256), 256, 0, st>>>(nl, leaves, dptr<int64_t>(LS.ent_ptr), cn, chunk, fib, fpb,
                                             dptr<AItem>(A.fw_items), ffirst);
   A.fw_first = ffirst;
   A.fw_part = nfp;
   // ---- transposition of the segments
-  HSR_HIP(dbuf_reserve(A.seg, sizeof(int32_t) * 6 * (ns + 2) + sizeof(int64_t) * 3 * (ns + 2) +
+  HSR_HIP(reserve(A.seg, sizeof(int32_t) * 6 * (ns + 2) + sizeof(int64_t) * 3 * (ns + 2) +
                                   sizeof(int32_t) * (n + 1)));
   int32_t *seg_t = dptr<int32_t>(A.seg);
   int32_t *key = seg_t + (ns + 2), *val = key + (ns + 2), *key2 = val + (ns + 2), *val2 = key2 + (ns + 2);
@@ -1026,7 +1031,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   while (bits < 31 && ((int64_t)1 << bits) <= 2 * nn + 1) ++bits;
   size_t tmp = 0;
   HSR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key2, val, val2, (int)ns, 0, bits, st));
-  HSR_HIP(dbuf_reserve(c->s.cub, tmp + 256));
+  HSR_HIP(reserve(c->s.cub, tmp + 256));
   HSR_HIP(hipcub::DeviceRadixSort::SortPairs(c->s.cub.p, tmp, key, key2, val, val2, (int)ns, 0, bits, st));
   A.key = key2;
   A.val = val2;
@@ -1040,8 +1045,8 @@ hsr_status adjoint_plan(hsr_ctx *c) {
     const bool fits = wbytes <= A.W.bytes || (double)wbytes <= 0.7 * (double)free_b;
     const int mode = c->tuning.adjoint_mode;
     A.fused = mode == 1 || (mode == 0 && fits);
-    if (A.fused) HSR_HIP(dbuf_reserve(A.W, wbytes));
-    HSR_HIP(dbuf_reserve(A.counts, sizeof(int64_t) * 4));
+    if (A.fused) HSR_HIP(reserve(A.W, wbytes));
+    HSR_HIP(reserve(A.counts, sizeof(int64_t) * 4));
   }
   if (!A.fused) {
     k_tr_counts<<<nblk(ns, 256), 256, 0, st>>>(ns, nn, key2, val2, seg_t, cn, leaves, tcnt, start);
@@ -1065,11 +1070,11 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   A.nruns = nruns;
   A.run_first = run_first;
   if (!A.fused) {
-    HSR_HIP(dbuf_reserve(A.tj, sizeof(int32_t) * (ntj + 1)));
+    HSR_HIP(reserve(A.tj, sizeof(int32_t) * (ntj + 1)));
     if (nsp) k_tr_expand<<<(unsigned)nsp, 64, 0, st>>>(nsp, val2, seg_t, cn, leaves, eoff, dptr<int32_t>(A.tj));
   }
   // source-pass items (two-pass schedule)
-  HSR_HIP(dbuf_reserve(A.tr, sizeof(int64_t) * 5 * (nruns + 2)));
+  HSR_HIP(reserve(A.tr, sizeof(int64_t) * 5 * (nruns + 2)));
   int64_t *tnc = dptr<int64_t>(A.tr), *tib = tnc + (nruns + 2), *tps = tib + (nruns + 2);
   int64_t *tpb = tps + (nruns + 2), *tfirst = tpb + (nruns + 2);
   if (nruns && !A.fused) {
@@ -1080,7 +1085,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
     const int64_t acc_p = tail_sum(c, tpb, tps, nruns);
     A.n_tr_items = acc_i;
     A.tr_part = acc_p;
-    HSR_HIP(dbuf_reserve(A.tr_items, sizeof(AItem) * (acc_i + 1)));
+    HSR_HIP(reserve(A.tr_items, sizeof(AItem) * (acc_i + 1)));
     k_tr_items_fill<<<nblk(nruns, 256), 256, 0, st>>>(nruns, nsp, run_first, key2, eoff, tcnt, cn, chunk, tnc,
                                                       tib, tpb, dptr<AItem>(A.tr_items), tfirst);
     tail_items[0] = acc_i;
@@ -1094,7 +1099,7 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   tail_items[1] = A.n_fw_items;
   HSR_HIP(hipMemcpyAsync(ffirst + nl, &tail_items[1], sizeof(int64_t), hipMemcpyHostToDevice, st));
   // canonical parents (for the pseudo push-down)
-  HSR_HIP(dbuf_reserve(A.par, sizeof(int32_t) * (nn + 1) + sizeof(int64_t) * (T.nboxes + 1)));
+  HSR_HIP(reserve(A.par, sizeof(int32_t) * (nn + 1) + sizeof(int64_t) * (T.nboxes + 1)));
   int32_t *par = dptr<int32_t>(A.par);
   int64_t *cb = reinterpret_cast<int64_t *>(par + nn + 1);
   HSR_HIP(hipMemcpyAsync(cb, T.box_root.data(), sizeof(int64_t) * (T.nboxes + 1), hipMemcpyHostToDevice, st));
@@ -1106,12 +1111,24 @@ hsr_status adjoint_plan(hsr_ctx *c) {
   HSR_HIP(hipStreamSynchronize(st));
   HSR_HIP(hipGetLastError());
   // buffers of the passes (reserved here so that a captured graph allocates nothing)
-  HSR_HIP(dbuf_reserve(A.qctr, sizeof(unsigned long long) * QWORDS));
-  HSR_HIP(dbuf_reserve(A.part, sizeof(float) * (std::max(A.fw_part, A.tr_part) + 1)));
-  HSR_HIP(dbuf_reserve(A.H, sizeof(float) * 3 * (nn + 1) + sizeof(float) * 3 * (A.npseudo + 1)));
+  HSR_HIP(reserve(A.qctr, sizeof(unsigned long long) * QWORDS));
+  HSR_HIP(reserve(A.part, sizeof(float) * (std::max(A.fw_part, A.tr_part) + 1)));
+  HSR_HIP(reserve(A.H, sizeof(float) * 3 * (nn + 1) + sizeof(float) * 3 * (A.npseudo + 1)));
   A.gen = c->lists_gen;
   A.planned_mode = c->tuning.adjoint_mode;
   return HSR_OK;
+}
+
+hsr_status adjoint_plan(hsr_ctx *c) {
+  const int64_t chunk = c->lists.chunk > 0 ? c->lists.chunk : 16384;
+  bool full = false;
+  hsr_status s = adjoint_plan_chunk(c, chunk, &full);
+  // the finer cut that the force phase takes by itself has no room here
+  if (s != HSR_OK && full && c->tuning.chunk == 0 && chunk < CHUNK_MAX) {
+    for (DBuf *b : {&c->adj.fw_items, &c->adj.tr_items, &c->adj.part}) dbuf_free(*b);
+    s = adjoint_plan_chunk(c, CHUNK_MAX, &full);
+  }
+  return s;
 }
 
 static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,

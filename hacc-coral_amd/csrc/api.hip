@@ -477,6 +477,7 @@ hipError_t dbuf_reserve(DBuf &b, size_t bytes) {
     e = hipMalloc(&b.p, want);
   }
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here: not again by the next check
     b.p = nullptr;
     return e;
   }

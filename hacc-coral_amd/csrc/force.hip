@@ -810,7 +810,7 @@ std::string force_shapes_built() {
 // 50^3 Plummer mix with leaves of 128; 0.87 and 0.47 ms (leaf kernel) at 64^3.
 // The partial sums the cut makes (12 bytes per target and item of a leaf
 // with several) stay below PART_MAX bytes.
-constexpr int64_t CHUNK_MAX = 8192, CHUNK_MIN = 256, ITEMS_PER_CU = 160;
+constexpr int64_t CHUNK_MIN = 256, ITEMS_PER_CU = 160;
 constexpr int64_t PART_MAX = (int64_t)1 << 28;
 
 static int64_t auto_chunk(const hsr_ctx *c) {
@@ -822,19 +822,32 @@ static int64_t auto_chunk(const hsr_ctx *c) {
   return chunk;
 }
 
-static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk);
+// (full: an allocation found no room)
+static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk, bool *full);
 
 hsr_status force_plan(hsr_ctx *c) {
-  if (c->tuning.chunk > 0) return force_plan_chunk(c, c->tuning.chunk);
+  bool full = false;
+  if (c->tuning.chunk > 0) return force_plan_chunk(c, c->tuning.chunk, &full);
   const int64_t chunk = auto_chunk(c);
-  hsr_status s = force_plan_chunk(c, chunk);
-  // a cap on the plan's memory that the finer cut exceeds
-  if (s == HSR_ERR_NOMEM && chunk < CHUNK_MAX) s = force_plan_chunk(c, CHUNK_MAX);
+  hsr_status s = force_plan_chunk(c, chunk, &full);
+  // what the finer cut takes more may exceed the caller's cap or the device
+  if (s != HSR_OK && chunk < CHUNK_MAX && (s == HSR_ERR_NOMEM || full)) {
+    if (full) {
+      dbuf_free(c->lists.items);
+      dbuf_free(c->lists.part);
+    }
+    s = force_plan_chunk(c, CHUNK_MAX, &full);
+  }
   return s;
 }
 
-static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
+static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk, bool *full) {
   hipStream_t st = c->stream;
+  auto reserve = [full](DBuf &b, size_t bytes) {
+    const hipError_t e = dbuf_reserve(b, bytes);
+    *full = e == hipErrorOutOfMemory;
+    return e;
+  };
   ListState &LS = c->lists;
   const int64_t nl = LS.nleaves;
   LS.chunk = chunk;
@@ -849,7 +862,7 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   // so their addresses (held by a captured force phase) survive list builds
   if (nl + 3 > LS.plan_stride) LS.plan_stride = std::max<int64_t>(nl + 3, LS.plan_stride + LS.plan_stride / 4);
   const int64_t ps = LS.plan_stride;
-  HSR_HIP(dbuf_reserve(LS.plan, sizeof(int64_t) * 8 * ps + sizeof(int32_t) * ps + 256));
+  HSR_HIP(reserve(LS.plan, sizeof(int64_t) * 8 * ps + sizeof(int32_t) * ps + 256));
   int64_t *nitem = dptr<int64_t>(LS.plan);
   int64_t *item_base = nitem + ps;
   int64_t *mflag = item_base + ps;
@@ -887,9 +900,9 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   }
   LS.nitems = nitems;
   LS.nmulti = nmulti;
-  HSR_HIP(dbuf_reserve(LS.items, sizeof(Item) * 2 * (nitems + 1)));
-  HSR_HIP(dbuf_reserve(LS.item_keys, sizeof(uint32_t) * 2 * NCLASS));
-  HSR_HIP(dbuf_reserve(LS.part, sizeof(float) * std::max<int64_t>(npart, 1)));
+  HSR_HIP(reserve(LS.items, sizeof(Item) * 2 * (nitems + 1)));
+  HSR_HIP(reserve(LS.item_keys, sizeof(uint32_t) * 2 * NCLASS));
+  HSR_HIP(reserve(LS.part, sizeof(float) * std::max<int64_t>(npart, 1)));
   Item *items_tmp = dptr<Item>(LS.items) + (nitems + 1);
   Item *items = dptr<Item>(LS.items);
   uint32_t *hist = dptr<uint32_t>(LS.item_keys);
@@ -904,7 +917,7 @@ static hsr_status force_plan_chunk(hsr_ctx *c, int64_t chunk) {
   LS.leaf_nchunk = nchunk;
   // target order inside the listed leaves
   const int64_t n = c->tree.n;
-  HSR_HIP(dbuf_reserve(LS.iperm, sizeof(int32_t) * std::max<int64_t>(n, 1)));
+  HSR_HIP(reserve(LS.iperm, sizeof(int32_t) * std::max<int64_t>(n, 1)));
   int32_t *iperm = dptr<int32_t>(LS.iperm);
   if (n) k_iota32<<<nblk(n, 256), 256, 0, st>>>(n, iperm);
   if (!c->tuning.tree_order_targets)

@@ -255,6 +255,9 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes,
 hsr_status lists_build_device(hsr_ctx *c, const float *min_force,
                               const float *max_force);
 hsr_status force_plan(hsr_ctx *c);
+// entries per work item where the caller sets none and the lists fill the
+// chip; where the finer cut of shorter lists has no room, too
+constexpr int64_t CHUNK_MAX = 8192;
 // where the force phase's pair totals (evaluated, unmasked) lie in its work
 // queue's buffer (s.qctr, in 8-byte words)
 constexpr int FORCE_TOTALS = 1024;
