@@ -625,7 +625,11 @@ hsr_status excl_scan(hsr_ctx *c, const T *in, T *out, int64_t n) {
 // divisions per pair.  The pair is bound by VALU issue: 16 FMA and a square
 // root in place of these took the leaf kernel from 6.88 to 1.00 ms on a
 // 60^3 Plummer mix (216k particles, leaves of 128, 3.1e8 pairs).
-void fit_poly(float *out, float *scale) {
+struct FitPoly {
+  float c[FITN + 1], scale;
+};
+
+FitPoly fit_poly() {
   const double b = 0.72f, cc = 0.01f, d = 0.27f, e = 0.0001f, ff = 360.0f, g = 100.0f, h = 0.67f,
                l = 17.0f, rmax = 3.116326355f;
   auto fgor = [&](double r) {
@@ -664,13 +668,15 @@ void fit_poly(float *out, float *scale) {
       tc[i] = tn[i];
     }
   }
-  for (int i = 0; i < n; ++i) out[i] = (float)mono[i];
-  *scale = (float)(2.0 / rmax);
+  FitPoly P;
+  for (int i = 0; i < n; ++i) P.c[i] = (float)mono[i];
+  P.scale = (float)(2.0 / rmax);
+  return P;
 }
 
 // P(r2) = sum a_k r2^k re-expanded in s = r2 + eps2 (host, double).
 LawArgs law_args(const ForceLawDev &D) {
-  LawArgs A;
+  LawArgs A = {};
   double a[7] = {0, 0, 0, 0, 0, 0, 0}, b[7] = {0, 0, 0, 0, 0, 0, 0};
   for (int k = 0; k <= 6; ++k) a[k] = D.c[k];
   const double e = D.eps2;
@@ -702,7 +708,11 @@ LawArgs law_args(const ForceLawDev &D) {
   A.in2 = (float)((double)D.rc2 * (1.0 - 1e-4));
   A.unmasked = D.guard ? 0 : 1;
   A.rc2 = D.rc2;
-  fit_poly(A.fit, &A.fit_a);
+  if (D.kind == LAWK_FIT) {
+    static const FitPoly P = fit_poly();  // of constants alone (3 us)
+    std::copy(P.c, P.c + FITN + 1, A.fit);
+    A.fit_a = P.scale;
+  }
   A.bins = D.bins;
   A.t_r2min = D.t_r2min;
   A.t_r2max = D.t_r2max;
