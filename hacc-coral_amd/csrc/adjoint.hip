@@ -374,6 +374,12 @@ __device__ __forceinline__ void fused_slice(const AdjLaw &L, float4 *pa, int tg,
                                             const float (&lb)[FR], const float (&lc)[FR],
                                             float (&am)[FR], float (&bx)[FR], float (&by)[FR],
                                             float (&bz)[FR]) {
+  // The whole wave's loop, where full passes spend their time, is put out of
+  // line with three others, which this moves too.  0 .. 7, fused adjoint of
+  // 256^3 with leaves of 512: 487.9, 473.7, 460.6, 474.4, 474.6, 483.4, 475.0
+  // and 490.6 ms (order 5), 497.2, 514.3, 501.6, 502.7, 481.0, 515.3, 485.7
+  // and 512.5 ms (order 6).
+  if constexpr (LP == 64) loop_offset<ORDER == 6 ? 4 : 2>();
   for (int k = 0; k < tg; k += FUNROLL) {
     float4 a[FUNROLL];
 #pragma unroll

@@ -348,6 +348,10 @@ k_force(const hsr_node *__restrict__ cn, const int32_t *__restrict__ leaves,
         __syncthreads();
         {
           const float4 *tp = tile + g * stride;
+          // 0 .. 7: 152.5, 154.1, 152.8, 155.3, 152.6, 154.4, 151.7 and 155.4 ms
+          // for shape (2, 2, 128), 151.3, 153.4, 151.7, 154.9, 151.8, 153.5,
+          // 151.1 and 154.9 for (2, 2, 256) (256^3, leaves of 512)
+          loop_offset<6>();
           for (int k = 0; k < tA; k += UNROLL) {
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {

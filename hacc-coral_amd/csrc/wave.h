@@ -15,6 +15,17 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
+// N instructions past a multiple of 32 bytes, for the code that follows.  The
+// time of a VALU-bound loop depends on where it starts modulo 32 bytes: moved
+// in steps of 4 bytes, the same instructions took 151.5 to 155.9 ms (k_force's
+// pair loops, 256^3), 461 to 491 ms (the fused adjoint's), the same again
+// after 32 bytes.  Any edit of a kernel moves its loops, so the hot ones say
+// where they start; each N was measured.
+template <int N>
+__device__ __forceinline__ void loop_offset() {
+  asm volatile(".p2align 5\n\t.rept %c0\n\ts_nop 0\n\t.endr" ::"i"(N));
+}
+
 // Exact, order-independent reductions (integer min / max / sum, float min /
 // max) by DPP: an inclusive scan within each row of 16 lanes (row_shr 1, 2,
 // 4, 8), then row 0's total into row 1 and row 2's into row 3 (row_bcast
