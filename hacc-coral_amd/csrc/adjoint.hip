@@ -309,7 +309,7 @@ k_adj_reduce(const hsr_node *cn, const AItem *items, const int64_t *first,
   const int64_t i0 = first[k], i1 = first[k + 1];
   if (i1 - i0 <= 1) return;  // single-chunk items wrote their result directly
   const hsr_node &nd = cn[items[i0].leaf];
-  for (int64_t i = threadIdx.x; i < nd.count; i += 256) {
+  for (int64_t i = threadIdx.x; i < nd.count; i += blockDim.x) {
     float sx = 0.f, sy = 0.f, sz = 0.f;
 #pragma unroll 4
     for (int64_t c = i0; c < i1; ++c) {
@@ -638,9 +638,9 @@ k_adj_fused6(HSR_ADJ_FUSED_ARGS) {
 // Fused schedule, source side: a workgroup per source leaf (a run of sorted
 // particle segments); particle k of the leaf receives m_k times the sum, over
 // the run's segments in sorted order, of W at the segment's entry for k.
-// Latency-bound: three dependent loads a segment before W's, so four waves
-// take the leaf's particles side by side and four segments are in flight (a
-// wave a leaf, a segment at a time: 1.85 ms at 128^3, now 0.95).
+// Latency-bound: three dependent loads a segment before W's, so a leaf's
+// particles are taken side by side (leaf_threads) and four segments are in
+// flight (a wave a leaf, a segment at a time: 1.85 ms at 128^3, now 0.95).
 __global__ void __launch_bounds__(256)
 k_src_reduce(int64_t nruns, int64_t nsp, const int64_t *__restrict__ run_first,
              const int32_t *__restrict__ key, const int32_t *__restrict__ val,
@@ -654,7 +654,7 @@ k_src_reduce(int64_t nruns, int64_t nsp, const int64_t *__restrict__ run_first,
   const int64_t p0 = run_first[r];
   const int64_t p1 = (r + 1 < nruns) ? run_first[r + 1] : nsp;
   const hsr_node &S = cn[key[p0]];
-  for (int64_t k = threadIdx.x; k < S.count; k += 256) {
+  for (int64_t k = threadIdx.x; k < S.count; k += blockDim.x) {
     float sx = 0.f, sy = 0.f, sz = 0.f;
 #pragma unroll 4
     for (int64_t p = p0; p < p1; ++p) {
@@ -1249,7 +1249,7 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
       LA(0, 5, dptr<AItem>(A.fw_items), counts);
     }
     if (A.fw_part)
-      k_adj_reduce<<<(unsigned)A.n_fw_leaves, 256, 0, st>>>(cn, dptr<AItem>(A.fw_items), A.fw_first,
+      k_adj_reduce<<<(unsigned)A.n_fw_leaves, leaf_threads(c), 0, st>>>(cn, dptr<AItem>(A.fw_items), A.fw_first,
                                                             A.n_fw_leaves, 0, A.fused ? iperm : nullptr,
                                                             part, gx, gy, gz);
   }
@@ -1260,7 +1260,7 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
   const int64_t ne = c->lists.nentries + 1;
   // source side of the fused schedule
   if (A.fused && A.nruns)
-    k_src_reduce<<<(unsigned)A.nruns, 256, 0, st>>>(A.nruns, A.nsp, A.run_first, A.key, A.val, A.seg_t, ent_ptr,
+    k_src_reduce<<<(unsigned)A.nruns, leaf_threads(c), 0, st>>>(A.nruns, A.nsp, A.run_first, A.key, A.val, A.seg_t, ent_ptr,
                                                   seg_e, cn, pj, W, W + ne, W + 2 * ne, gx, gy, gz);
   // source pass of the two-pass schedule
   if (!A.fused && A.n_tr_items) {
@@ -1270,7 +1270,7 @@ static hsr_status adjoint_enqueue(hsr_ctx *c, const float *lx, const float *ly,
     else LA(1, 5, dptr<AItem>(A.tr_items), counts + 1);
 #undef LA
     if (A.tr_part)
-      k_adj_reduce<<<(unsigned)A.n_tr_leaves, 256, 0, st>>>(cn, dptr<AItem>(A.tr_items), A.tr_first,
+      k_adj_reduce<<<(unsigned)A.n_tr_leaves, leaf_threads(c), 0, st>>>(cn, dptr<AItem>(A.tr_items), A.tr_first,
                                                             A.n_tr_leaves, 1, nullptr, part, gx, gy, gz);
   }
   // pseudo pass

@@ -258,6 +258,15 @@ hsr_status force_plan(hsr_ctx *c);
 // entries per work item where the caller sets none and the lists fill the
 // chip; where the finer cut of shorter lists has no room, too
 constexpr int64_t CHUNK_MAX = 8192;
+// Threads of a workgroup that sums for a leaf's particles side by side, a
+// particle a thread: the waves that leaves of nd particles fill.  k_src_reduce
+// with 64, 128 and 256 threads: 35.1, 53.3 and 53.4 ms (64^3, nd 8), 4.07,
+// 5.56 and 5.63 (nd 32), 1.83, 1.84 and 1.83 (nd 64), 1.74, 0.87 and 0.88 (nd
+// 128), 2.98, 2.20 and 1.75 (128^3, nd 200): waves without a particle cost as
+// much to start and to drain as those with one.
+inline unsigned leaf_threads(const hsr_ctx *c) {
+  return c->p.nd <= 64 ? 64 : c->p.nd <= 128 ? 128 : 256;
+}
 // where the force phase's pair totals (evaluated, unmasked) lie in its work
 // queue's buffer (s.qctr, in 8-byte words)
 constexpr int FORCE_TOTALS = 1024;
