@@ -1514,10 +1514,26 @@ __global__ void k_box_of(const BNode *nodes, int64_t nb, int32_t *box_of) {
 // particles.  Build time without and with it: 0.99 and 0.63 ms for 12k
 // particles (leaves of 32), 1.93 and 1.62 ms for 365k (leaves of 128), but
 // 3.95 and 4.10 ms for 2.5M (leaves of 256), 9.78 and 10.58 ms for 18M.
-constexpr int SUB_T = 1024;
+//
+// Leaves of one to three particles give a subtree levels of hundreds of nodes,
+// 16 waves for all of them, and a middle-sized build too few subtrees to hide
+// that.  Without and with it, leaves of 1: 0.69 and 0.42 ms for 300 particles,
+// 0.79 and 0.71 for 700, 0.81 and 0.92 for 1000, 0.95 and 1.65 for 2000, 1.71
+// and 2.18 for 32000, 1.95 and 1.99 for 48000, 2.23 and 2.18 for 64000; leaves
+// of 2: 0.81 and 0.87 ms for 1500, 1.54 and 1.74 for 32000, 1.69 and 1.63 for
+// 48000; of 3: 0.83 and 0.91 for 2000, 1.42 and 1.50 for 32000; of 4: 0.78
+// and 0.78 for 2000, 1.39 and 1.35 for 32000.
 constexpr int64_t SUB_N = (int64_t)1 << 20;
-constexpr int SUB_LEVELS = SUB_MAX;  // every level but a subtree's first follows a
-                                     // split, which takes a particle off its node
+
+inline bool subtrees_pay(int64_t n, int64_t nd) {
+  return n <= SUB_N && (nd > 3 || n <= 512 * nd || n > 56000);
+}
+
+constexpr int SUB_T = 1024;
+// Every level but a subtree's first follows a split, which takes a particle
+// off its node.  (Tables for 48 levels, a deeper tree built again by the level
+// passes: 5.0 ms for 285 particles in 62 levels, 1.75 now, 3.7 by the passes.)
+constexpr int SUB_LEVELS = SUB_MAX;
 
 struct SubCtr {
   int64_t next;      // next free node slot
@@ -2316,7 +2332,7 @@ hsr_status tree_build_device(hsr_ctx *c, int64_t nboxes, const int64_t *box_off_
   int64_t active = n;
   Counters hc;
   int depth = 0;
-  const bool use_sub = unit && n <= SUB_N;
+  const bool use_sub = unit && subtrees_pay(n, nd);
   // whether the level holds nodes above CM_SMALL, up to it, and leaves for the
   // level passes to finish (with subtrees, k_subtree takes all up to SUB_MAX)
   bool run_big = false, run_small = !use_sub, run_leaf = true;
