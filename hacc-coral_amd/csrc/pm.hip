@@ -484,6 +484,16 @@ __device__ __forceinline__ void merge_advance(int qs, int32_t (&s)[8], const int
     }
 }
 
+// What the host reads, in one copy: the outside slot's contributions, and
+// whether the keys are out of order.
+__global__ void k_cic_totals(const int32_t *out_last, const int32_t *nout_last, const int32_t *unsorted,
+                             int64_t *totals) {
+  if (threadIdx.x == 0) {
+    totals[0] = (int64_t)*out_last + *nout_last;
+    totals[1] = *unsorted;
+  }
+}
+
 // The corners in the order of their base cells' keys, for any cell: with the
 // particles in base-cell order (k_cic_base) a cell's contributions are its
 // eight lists one after another in this order.
@@ -869,7 +879,7 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   // run key; the long-cell counter
   const size_t nn = (size_t)n, nc = (size_t)g.safe, ms = 8 * nn, ne = (size_t)ex.out;
   // (each array starts on a 256-byte boundary: 14 arrays)
-  const size_t bytes = 8 * (nc + ms) + 4 * (6 * nn + 2 * ne + nc + ms) + 16 + 14 * 256;
+  const size_t bytes = 8 * (nc + ms) + 4 * (6 * nn + 2 * ne + nc + ms) + 32 + 14 * 256;
   HSR_HIP(dbuf_reserve(c->sub.keys, bytes));
   char *bp = (char *)c->sub.keys.p;
   auto take = [&bp](size_t b) {
@@ -889,7 +899,7 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   int32_t *end = (int32_t *)take(4 * ne);
   uint32_t *long_cell = (uint32_t *)take(4 * nc);
   uint32_t *skey = (uint32_t *)take(4 * ms);
-  unsigned long long *nlong = (unsigned long long *)take(16);  // and the unsorted flag
+  unsigned long long *nlong = (unsigned long long *)take(32);  // and the unsorted flag, the host's totals
   int32_t *unsorted = (int32_t *)(nlong + 1);
   if ((size_t)(bp - (char *)c->sub.keys.p) > c->sub.keys.bytes) {
     hsr_set_error("hsr_cic: staging layout exceeds its buffer");
@@ -903,17 +913,17 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   // one host round trip, which the contributions' count takes anyway
   hsr_status s;
   if ((s = pm_excl_scan(c, nout, out_base, n)) != HSR_OK) return s;
-  int32_t last[3] = {0, 0, 0};
-  HSR_HIP(hipMemcpyAsync(&last[0], out_base + n - 1, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&last[1], nout + n - 1, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  HSR_HIP(hipMemcpyAsync(&last[2], unsorted, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  int64_t *totals = (int64_t *)(nlong + 2);
+  k_cic_totals<<<1, 64, 0, st>>>(out_base + n - 1, nout + n - 1, unsorted, totals);
+  int64_t last[2] = {0, 0};
+  HSR_HIP(hipMemcpyAsync(last, totals, sizeof(last), hipMemcpyDeviceToHost, st));
   HSR_HIP(stream_wait(st));
-  const int64_t m = (int64_t)last[0] + last[1];
+  const int64_t m = last[0];
   if ((size_t)m > ms) {
     hsr_set_error("hsr_cic: staged contributions exceed 8 per particle");
     return HSR_ERR_STATE;
   }
-  if (last[2]) {
+  if (last[1]) {
     size_t tmp = 0;
     HSR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key2, idx, idx2, (int)n, 0, bits, st));
     HSR_HIP(dbuf_reserve(c->s.cub, tmp + 256));
@@ -930,11 +940,11 @@ hsr_status cic_run(hsr_ctx *c, int64_t n, const float *x, const float *y, const 
   k_cic_ranges<<<nblk(n, 256), 256, 0, st>>>(n, key2, ex, beg, end);
   // short cells summed, long ones queued and summed a workgroup each (the
   // grid loops over the device-side count)
-  const auto cells = last[2] ? &k_cic_cells<false> : &k_cic_cells<true>;
+  const auto cells = last[1] ? &k_cic_cells<false> : &k_cic_cells<true>;
   cells<<<nblk((int64_t)nc, 256), 256, 0, st>>>(g, ex, beg, end, idx2, x, y, z, cc, rho, long_cell, long_k,
                                                 nlong);
   const unsigned lgrid = (unsigned)std::max(1, c->num_cus) * 32;
-  const auto long_sum = last[2] ? &k_cic_long_sum<false> : &k_cic_long_sum<true>;
+  const auto long_sum = last[1] ? &k_cic_long_sum<false> : &k_cic_long_sum<true>;
   long_sum<<<lgrid, 64, 0, st>>>(g, ex, beg, end, idx2, long_cell, long_k, nlong, x, y, z, cc, rho);
   // the outside slot: its contributions in (particle, corner) order
   if (m > 0) {
