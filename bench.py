@@ -36,8 +36,9 @@ PEAK_HBM_GBPS = 8000.0       # MI355X HBM3E
 # figure is reported only for the build it was measured on.
 MEASURED_TRAFFIC = {
     # profiles/k_force_256c_traffic.md
-    ("B", 256, 512, 1, (2, 2, 128), "ba11f51afafb0511"): 144144650880,
-    ("B", 256, 640, 1, (2, 2, 128), "ba11f51afafb0511"): 147090420416,
+    ("B", 256, 384, 1, (2, 2, 256), "b059f4a3063bb81e"): 145522398528,
+    ("B", 256, 512, 1, (2, 2, 128), "b059f4a3063bb81e"): 137966162272,
+    ("B", 256, 640, 1, (2, 2, 256), "b059f4a3063bb81e"): 137203530944,
 }
 
 
@@ -350,9 +351,9 @@ def pm_leg(load, dev, reps=3):
             "inverse_cic": {"ms": i_ms, "algorithmic_bytes": ib,
                             "GB/s": ib / (i_ms * 1e-3) / 1e9,
                             "frac": ib / (i_ms * 1e-3) / 1e9 / PEAK_HBM_GBPS},
-            "note": "deposit bit-exact with the reference's sequential float order: particles "
-                    "sorted by base cell, each cell's eight neighbour lists merged by particle "
-                    "index and its terms added in that order"}
+            "note": "deposit bit-exact with the reference's sequential float order: each cell's "
+                    "terms added in particle order from its eight base cells' lists (the "
+                    "particles sorted by base cell where they are not in that order already)"}
 
 
 def refresh_leg(load, dev, reps=3):

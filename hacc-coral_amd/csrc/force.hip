@@ -746,11 +746,11 @@ __global__ void k_iota32(int64_t n, int32_t *a) {
 
 // Every target's place is the number of smaller keys in its leaf: n broadcast
 // LDS reads a target and no barriers, where a bitonic sort took log^2 n of
-// them (0.68 -> 0.41 ms at 256^3 with leaves of 512).  The keys
-// are whole coordinates: their leading 22 bits alone leave dense leaves
-// unordered and widen their passes' boxes (fused adjoint 474 ms at 256^3 in
-// the tree that had them, 455 with the bitonic sort; not timed since, and
-// the 0.41 ms are of the shorter keys).
+// them (0.70 -> 0.53 ms at 256^3 with leaves of 512).  The keys are whole
+// coordinates: their leading 22 bits, with the position in the other ten, took
+// 0.41 ms, but leave targets that agree in them in tree order (evaluated pairs
+// 4.1216e11 against 4.1205e11 there, 0.03%: 0.05 ms of the leaf kernel, and
+// three times that of the adjoint).
 __global__ void __launch_bounds__(256)
 k_leaf_sort(int64_t nl, const int32_t *__restrict__ leaves, const hsr_node *__restrict__ cn,
             const PJ *__restrict__ pj, int32_t *__restrict__ iperm) {

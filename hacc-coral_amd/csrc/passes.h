@@ -15,6 +15,11 @@
 // Against powers of two down to 8 and then the rest: leaf kernel 0.40 ->
 // 0.35 ms at 61^3 (quadrupole, leaves of 100), 0.033 -> 0.020 ms at 16^3
 // (leaves of 32), 8.77 -> 8.53 ms for 24 boxes of 20^3..64^3 (leaves of 256).
+// The fused adjoint takes the same passes, though its pairs cost three times
+// as much beside the staging.  Powers of two and this rule there: 0.21 and 0.19
+// ms at 16^3 (leaves of 32), 0.26 and 0.25 at 32^3 (50), 12.12 and 11.84 at
+// 64^3 (64), 10.82 and 10.79 (100), 61.5 and 62.2 at 128^3 (100), 453.4 and
+// 455.5 at 256^3 (384), each with its hot loop at its best place (loop_offset).
 template <int R>
 __host__ __device__ inline int pass_slots(int64_t rem, int pmax, bool thin) {
   if (rem >= pmax) return pmax;

@@ -13,10 +13,12 @@
 // with one load before it moves, and gives a counter up for good when a pop
 // comes back past its end, so at most QN pops per wave fail and every wave
 // leaves.  Item i belongs to counter i % QN; runs of 8 or 32 consecutive
-// items per counter, which keep neighbouring leaves in one XCD's L2, were 2%
-// slower at 256^3 and no faster elsewhere.  Leaf kernel, one counter and
+// items per counter, which keep neighbouring leaves in one XCD's L2, were no
+// faster (2% slower at 256^3, which is what moving the pair loops by a few
+// bytes can do, see loop_offset in wave.h).  Leaf kernel, one counter and
 // now: 0.167 and 0.029 ms for 265 leaves of 32 (1155 entries each), 109.4
-// ms either way for 50k leaves of 512 at 256^3.
+// ms either way for 50k leaves of 512 at 256^3; fused adjoint of 256^3, each
+// with its loop at its best place, 458.7 and 460.4.
 #pragma once
 
 #include "wave.h"

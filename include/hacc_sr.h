@@ -422,8 +422,9 @@ typedef struct {
                          polynomial laws with rsm > 0; sums in another order:
                          rounding only */
   int tile;           /* j entries staged per LDS tile (0 = 256) */
-  int chunk;          /* maximum list entries per work item: 0 (= 8192) or
-                         tile..2^30; a change re-plans lists already built
+  int chunk;          /* maximum list entries per work item: 0 (8192, or where
+                         the lists give the chip too few items that way a
+                         power of two down to 256) or tile..2^30; a change re-plans lists already built
                          (on failure the old tuning and plan are restored
                          where possible; otherwise the lists must be built
                          again and calls that need them give HSR_ERR_STATE) */
@@ -446,7 +447,8 @@ typedef struct {
                          sums in another order: rounding only); 64 and 32
                          times i_per_lane in general */
   int64_t max_plan_bytes; /* cap on the device memory of the force plan (work
-                         items, their sort keys, chunk partials); 0: no cap.
+                         items, chunk partials); 0: no cap.  With chunk 0 a
+                         plan above it falls back to items of 8192 entries.
                          A plan above it fails with HSR_ERR_NOMEM before any
                          launch (so does one of 2^31 work items or more) */
   int unroll;         /* leaf kernel shape: j entries per unrolled step (0 = 2) */
