@@ -40,7 +40,7 @@ def test_deep_tree_is_built_once():
     for mass in (1.0, 0.5):  # one subtree; the passes over levels
         ctx = Context(nd=1)
         best = np.inf
-        for _ in range(4):
+        for _ in range(8):
             x, y, z = (p[:, k].copy() for k in range(3))
             ctx.build(x, y, z, np.full(p.shape[0], mass, np.float32), min_loc=(0, 0, 0), max_loc=(8, 8, 8))
             best = min(best, ctx.stats().build_ms)

